@@ -235,7 +235,10 @@ int srg_end_frame(srg_ctx* ctx);
 #define SRG_NOALLOC_TABLE_BYTES (256u << 10)
 int srg_end_frame_noalloc(srg_ctx* ctx);
 /* Copies the write plane's colour to linear RGBA8 rows (width*height*4 bytes),
- * swaps the planes, then calls on_finish(user) (Renderer.cpp:350-372). */
+ * swaps the planes, then calls on_finish(user) (Renderer.cpp:350-372).
+ * Page-locked memory (hipHostMalloc) is written by the GPU itself, at the
+ * host link's rate; pageable memory is written through page-locked chunks.
+ * The same holds for srg_blit_async. */
 int srg_blit(srg_ctx* ctx, srg_fb* fb, void* linear_rgba8, void (*on_finish)(void*), void* user);
 /* Blit (Renderer.cpp:350-372) with the reference's asynchrony: returns at
  * once; on a second stream the write plane is de-tiled into pinned memory
