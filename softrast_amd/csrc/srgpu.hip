@@ -256,6 +256,7 @@ struct srg_ctx {
     DevArray<uint32_t> blit_staging;    // rows for a blit to memory that is neither host allocation nor page-locked
     uint32_t* stage = nullptr;          // two page-locked chunks through which pageable memory is written (staged_out)
     hipEvent_t stage_ev[2] = {};
+    DevArray<uint8_t> tex_work;         // texture building: base image, filtered rows, weights
     uint32_t* h_counters = nullptr;
     uint32_t clip_cap = 0, entry_cap = 0;
     uint32_t last_bins = 0;
@@ -286,6 +287,9 @@ struct srg_ctx {
 
 namespace {
 
+// A texture workspace of at most this is kept for the context's next texture
+// (20 bytes a texel of the base level: up to 2048^2); a larger one is freed.
+constexpr size_t kTexWorkKeep = 96u << 20;
 constexpr size_t kStageBytes = 512u << 10;  // of each of srg_ctx::stage's two chunks
 
 uint64_t new_handle(srg_ctx* ctx) { return ctx->next_handle++; }
@@ -441,14 +445,14 @@ int staged_out(srg_ctx* ctx, void* dst, size_t units, size_t unit_bytes, Emit em
     return st;
 }
 
-// `words` 32-bit words of device memory to the caller's memory; ordered after
-// the library stream, done on return (page-locked and other memory: when the
-// stream is done).
+// `words` 32-bit words of device memory to the caller's memory, after the work
+// on the library stream; done on return.
 int copy_out(srg_ctx* ctx, void* dst, const uint32_t* src, size_t words)
 {
     uint32_t* dev;
     if (classify_dst(dst, words * 4, &dev) != HostDst::pageable) {
         HIP_TRY(hipMemcpyAsync(dst, src, words * 4, hipMemcpyDeviceToHost, ctx->stream));
+        HIP_TRY(hipStreamSynchronize(ctx->stream));
         return SRG_OK;
     }
     constexpr size_t unit = 1024;  // words
@@ -1457,6 +1461,7 @@ void srg_destroy(srg_ctx* ctx)
     ctx->bin_cost.release();
     ctx->counters.release();
     ctx->blit_staging.release();
+    ctx->tex_work.release();
     if (ctx->h_tables) (void)hipHostFree(ctx->h_tables);
     if (ctx->h_counters) (void)hipHostFree(ctx->h_counters);
     if (ctx->stage) (void)hipHostFree(ctx->stage);
@@ -1643,7 +1648,6 @@ int srg_fb_read_tiles(srg_ctx* ctx, srg_fb* fb, uint32_t plane, uint32_t* colour
         if (!p.primid) return SRG_ERR_INVALID;
         if ((st = copy_out(ctx, primid, p.primid, n))) return st;
     }
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
     return SRG_OK;
 }
 
@@ -2101,6 +2105,30 @@ static bool mitchell_resize_rgba8(const uint8_t* in, uint32_t w, uint32_t h, uin
     return true;
 }
 
+// The filters of scales 2^1 .. 2^smax as the device's passes read them
+// (mip_weights_at): the weights mitchell_axis gives every output, whose
+// offsets from its taps are the same for each (powers of two, exact in float).
+static void mip_filters(uint32_t smax, MipF4* out)
+{
+    std::vector<float> w;
+    for (uint32_t s = 1; s <= smax; ++s) {
+        const uint32_t n = 1u << s, taps = 4 * n;
+        const float scale = 1.0f / (float)n;
+        w.resize(taps);
+        // tap t of output 0 is input t - 1.5 n: the filter is even
+        for (uint32_t t = 0; t < taps / 2; ++t) {
+            const float c = ((float)t - 1.5f * (float)n) + 0.5f;
+            w[t] = w[taps - 1 - t] = mitchell(0.5f - c * scale) * scale;
+        }
+        float sum = 0.0f;
+        for (uint32_t t = 0; t < taps; ++t) sum += w[t];
+        const float inv = 1.0f / sum;
+        for (uint32_t t = 0; t < taps; ++t) w[t] *= inv;
+        for (uint32_t a = 0; a < n; ++a)
+            out[mip_weights_at(s) + a] = MipF4{ w[a], w[a + n], w[a + 2 * n], w[a + 3 * n] };
+    }
+}
+
 // Layout of CreateFromRGBA8 (Texture.cpp:119-177): power-of-two sizes, each
 // a multiple of the 32-texel tile and below 2^14; a full chain when mips are
 // made; every level padded to whole 32x32 tiles.
@@ -2165,79 +2193,65 @@ int srg_texture_create_rgba8(srg_ctx* ctx, const uint8_t* linear, uint32_t width
     if (!ctx || !out || !linear) return SRG_ERR_INVALID;
     int st = texture_layout(width, height, calc_mips, L);
     if (st) return st;
-    // per-level tap lists, built on the host before anything is allocated
-    std::vector<AxisTaps> tx(L.n), ty(L.n);
-    size_t ntaps = 0;
-    for (uint32_t m = 1; m < L.n; ++m) {
+    // the passes of every level, longest chains (highest levels) first
+    MipPasses px{}, py{};
+    uint32_t bx = 0, by = 0, smax = 0;
+    size_t nrows = 0;  // float4
+    uint64_t zero_at = L.total;  // the levels with padding texels, the last of the chain
+    for (uint32_t m = L.n; m-- > 1;) {
         const uint32_t mw = std::max(1u, width >> m), mh = std::max(1u, height >> m);
-        if (!mitchell_axis(width, mw, tx[m]) || !mitchell_axis(height, mh, ty[m])) return SRG_ERR_INVALID;
-        // words: first (n + 1), src and weight per axis
-        ntaps += tx[m].first.size() + 2 * tx[m].src.size() + ty[m].first.size() + 2 * ty[m].src.size();
+        if (mw < 32 || mh < 32) zero_at = L.offs[m];
+        auto pass = [&](MipPasses& P, uint32_t& block, uint32_t in_log2, uint32_t outs, uint32_t lines) {
+            MipPass& q = P.level[P.n++];
+            q.block = block;
+            q.log2_scale = in_log2 - (uint32_t)__builtin_ctz(outs);
+            q.out = outs;
+            q.lines = lines;
+            q.seg = std::max(1u, kMipSegTexels >> q.log2_scale);
+            q.segs = (outs + q.seg - 1) / q.seg;
+            q.rows_at = (uint32_t)nrows;
+            q.dst_at = L.offs[m] / 4;
+            block += q.segs * ((lines + 15) / 16);
+            smax = std::max(smax, q.log2_scale);
+        };
+        pass(px, bx, L.wl, mw, height);
+        pass(py, by, L.hl, mh, mw);
+        nrows += (size_t)height * mw;
     }
+    // one workspace: base image, rows, weights
+    const size_t base_bytes = (size_t)width * height * 4, w_count = smax ? mip_weights_at(smax + 1) : 0;
+    const size_t rows_at = base_bytes, weights_at = rows_at + nrows * 16, work = weights_at + w_count * 16;
     Texture t;
     t.bytes = L.total;
     t.wlog2 = L.wl;
     t.hlog2 = L.hl;
     t.nmips = L.n;
     std::memcpy(t.mip_offsets, L.offs, sizeof(L.offs));
-    uint32_t* base = nullptr;
-    float4* rows = nullptr;
-    uint8_t* taps = nullptr;
-    std::vector<uint8_t> htaps;
-    const size_t row_bytes = L.n > 1 ? sizeof(float4) * (size_t)height * std::max(1u, width >> 1) : 0;
     auto cleanup = [&](int code) {
         (void)hipStreamSynchronize(ctx->stream);
-        if (base) (void)hipFree(base);
-        if (rows) (void)hipFree(rows);
-        if (taps) (void)hipFree(taps);
+        if (ctx->tex_work.cap > kTexWorkKeep) ctx->tex_work.release();
         if (code && t.dev) (void)hipFree(t.dev);
         return code;
     };
-    if (hipMalloc((void**)&t.dev, L.total) != hipSuccess || hipMalloc((void**)&base, (size_t)width * height * 4) != hipSuccess ||
-        (row_bytes && hipMalloc((void**)&rows, row_bytes) != hipSuccess) ||
-        (ntaps && hipMalloc((void**)&taps, ntaps * 4) != hipSuccess))
-        return cleanup(SRG_ERR_NOMEM);
-    if (hipMemcpyAsync(base, linear, (size_t)width * height * 4, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
+    if (hipMalloc((void**)&t.dev, L.total) != hipSuccess) return SRG_ERR_NOMEM;
+    if ((st = ctx->tex_work.ensure(work))) return cleanup(st);
+    uint32_t* base = (uint32_t*)ctx->tex_work.ptr;
+    float* rows = (float*)(ctx->tex_work.ptr + rows_at);
+    MipF4* weights = (MipF4*)(ctx->tex_work.ptr + weights_at);
+    if (hipMemcpyAsync(base, linear, base_bytes, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
         return cleanup(SRG_ERR_HIP);
-    // all tap lists in one upload: per level first_x, src_x, w_x, first_y, src_y, w_y
-    htaps.resize(ntaps * 4);
-    std::vector<MipTaps> dx(L.n), dy(L.n);
-    size_t at = 0;
-    auto put = [&](const void* p, size_t words) {
-        const size_t o = at;
-        if (at + words <= ntaps) std::memcpy(htaps.data() + o * 4, p, words * 4);
-        at += words;
-        return o;
-    };
-    for (uint32_t m = 1; m < L.n; ++m) {
-        const size_t fx = put(tx[m].first.data(), tx[m].first.size()), sx = put(tx[m].src.data(), tx[m].src.size());
-        const size_t wx = put(tx[m].weight.data(), tx[m].weight.size());
-        const size_t fy = put(ty[m].first.data(), ty[m].first.size()), sy = put(ty[m].src.data(), ty[m].src.size());
-        const size_t wy = put(ty[m].weight.data(), ty[m].weight.size());
-        const uint32_t* T = (const uint32_t*)taps;
-        dx[m] = MipTaps{ T + fx, T + sx, (const float*)(T + wx) };
-        dy[m] = MipTaps{ T + fy, T + sy, (const float*)(T + wy) };
+    const uint32_t tiles_w = width >> 5, ntex = width * height, nzero = (uint32_t)((L.total - zero_at) / 4);
+    hipLaunchKernelGGL(k_tex_tile, dim3((ntex + nzero + 255) / 256), dim3(256), 0, ctx->stream, base, width,
+                       (uint32_t*)t.dev, tiles_w, ntex, (uint32_t*)(t.dev + zero_at), nzero);
+    std::vector<MipF4> hw(w_count);
+    if (L.n > 1) {
+        mip_filters(smax, hw.data());
+        if (hipMemcpyAsync(weights, hw.data(), w_count * 16, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
+            return cleanup(SRG_ERR_HIP);
+        hipLaunchKernelGGL(k_mip_rows, dim3(bx), dim3(64), 0, ctx->stream, base, width, px, weights, rows);
+        hipLaunchKernelGGL(k_mip_cols, dim3(by), dim3(64), 0, ctx->stream, rows, height, py, weights, (uint32_t*)t.dev);
     }
-    if (at != ntaps) return cleanup(SRG_ERR_INVALID);  // tap lists must fill the upload exactly
-    if (ntaps && hipMemcpyAsync(taps, htaps.data(), at * 4, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
-        return cleanup(SRG_ERR_HIP);
-    for (uint32_t m = 0; m < L.n; ++m) {
-        const uint32_t mw = std::max(1u, width >> m), mh = std::max(1u, height >> m);
-        const uint32_t tiles_w = (mw + 31u) >> 5, tiles_h = (mh + 31u) >> 5;
-        const uint32_t ntex = tiles_w * tiles_h * 1024u;
-        uint32_t* dst = (uint32_t*)(t.dev + L.offs[m]);
-        if (m == 0) {
-            hipLaunchKernelGGL(k_tex_tile, dim3((ntex + 255) / 256), dim3(256), 0, ctx->stream, base, width, height, dst,
-                               tiles_w, ntex);
-        } else {
-            hipLaunchKernelGGL(k_mip_rows, dim3((height * mw + 255) / 256), dim3(256), 0, ctx->stream, base, width, height,
-                               mw, dx[m], rows);
-            hipLaunchKernelGGL(k_mip_cols, dim3((ntex + 255) / 256), dim3(256), 0, ctx->stream, rows, mw, mh, dy[m], dst,
-                               tiles_w, ntex);
-        }
-        if (hipGetLastError() != hipSuccess) return cleanup(SRG_ERR_HIP);
-    }
-    if (hipStreamSynchronize(ctx->stream) != hipSuccess) return cleanup(SRG_ERR_HIP);
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ctx->stream) != hipSuccess) return cleanup(SRG_ERR_HIP);
     cleanup(SRG_OK);
     const uint64_t h = new_handle(ctx);
     ctx->textures[h] = t;
@@ -2262,10 +2276,8 @@ int srg_texture_read(srg_ctx* ctx, srg_handle h, uint8_t* out, uint64_t capacity
     if (t.bytes) {
         if (const int st = copy_out(ctx, out, (const uint32_t*)t.dev, t.bytes / 4)) return st;
         if (t.bytes % 4)
-            HIP_TRY(hipMemcpyAsync(out + t.bytes / 4 * 4, t.dev + t.bytes / 4 * 4, t.bytes % 4, hipMemcpyDeviceToHost,
-                                   ctx->stream));
+            HIP_TRY(hipMemcpy(out + t.bytes / 4 * 4, t.dev + t.bytes / 4 * 4, t.bytes % 4, hipMemcpyDeviceToHost));
     }
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
     return SRG_OK;
 }
 

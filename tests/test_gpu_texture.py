@@ -60,3 +60,19 @@ def test_draw_with_device_texture_same_image():
     for a, b in zip(ref[:3], out[:3]):
         assert np.array_equal(a, b)
     ctx.Shutdown()
+
+
+@pytest.mark.parametrize("w,h", [(32, 64), (32, 4096), (4096, 32), (512, 32), (64, 1024), (256, 512), (1024, 1024)])
+def test_device_mips_long_and_short_lines(w, h):
+    """Lines of one segment and of many, axes that reach one texel long before
+    the other (levels narrower than a wave's 16 columns, sums of every input
+    texel and its clamped edges), extreme bytes at the edges."""
+    import softrast_amd as sr
+    _say(f"[texture] case=device_mips size={w}x{h}")
+    img = np.random.default_rng(w * 8192 + h).integers(0, 256, (h, w, 4), dtype=np.uint8)
+    img[:, 0], img[:, -1], img[0], img[-1] = 255, 0, 255, 0
+    host = sr.TextureData().CreateFromRGBA8(img, w, h, True)
+    ctx = sr.RenderContext()
+    for _ in range(2):  # the second build works in the first one's workspace
+        assert np.array_equal(ctx.CreateTexture(img, w, h, True).read().m_texels, host.m_texels)
+    ctx.Shutdown()
