@@ -88,7 +88,7 @@ typedef struct srg_config {
     uint32_t tile_order;    /* srg_tile_order */
     uint32_t max_prims;     /* initial primitive-record capacity, 0 = sized per frame */
     uint32_t max_entries;   /* initial tile-entry capacity, 0 = sized per frame */
-    uint32_t wg_per_cu;     /* persistent back-end workgroups per CU, 0 = default */
+    uint32_t wg_per_cu;     /* persistent back-end workgroups per CU, at most (0 = as many as are resident) */
     uint32_t bin_size;      /* back-end work bin edge: 64, 32, 16 or 8 pixels, 0 = 32. The
                                reference's 64x64 bin semantics are kept for every size. */
     uint32_t sched_warmup_frames;    /* SRG_ORDER_LEARNED: frames recorded before the first

@@ -224,6 +224,7 @@ __device__ __forceinline__ uint32_t shade_pixel(const FrameDev& F, uint32_t rec,
 // a chain of dependent loads); more views are binary-searched.
 __device__ __forceinline__ uint32_t view_of_bin(const FrameDev& F, uint32_t gb)
 {
+    if (F.nviews == 1u) return 0u;
     if (F.nviews <= 64u) {
         const uint32_t lane = lane_id();
         const bool le = lane < F.nviews && F.views[lane].bin_base <= gb;
@@ -533,7 +534,7 @@ __global__ __launch_bounds__(backend_threads(S, H), backend_min_waves(S, H, STAT
     __shared__ unsigned long long keys[NPIX];
     __shared__ uint32_t s_stage[W * kStageWords];
     // the next queue item, handed to the workgroup through the first key slot
-    // (free between the end of one item's shading and its key initialisation)
+    // (free between the end of one item's shading and the next one's key initialisation)
     uint32_t& s_q = *(uint32_t*)&keys[0];
     const uint32_t tid = threadIdx.x, lane = tid & 63u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
@@ -543,12 +544,15 @@ __global__ __launch_bounds__(backend_threads(S, H), backend_min_waves(S, H, STAT
     // per-bin costs: requested, and (for the learned order) a recording frame
     const bool timed = (F.flags & FF_TILE_COSTS) && (!F.sched_gate || F.sched_gate[1]);
 
-    for (;;) {
-        if (tid == 0) s_q = atomicAdd(&F.counters[C_QHEAD], 1u);
-        __syncthreads();
-        const uint32_t qi = s_q;
-        __syncthreads();
-        if (qi >= qlen) break;
+    // Workgroup b's first item is item b; further ones come from the queue's
+    // counter, which only a queue longer than the grid needs. (Popping every
+    // item, each of 2,048 workgroups made an atomic on one address before its
+    // first item and one that found the queue empty: 15-35 us on any frame.
+    // Asking for the next item before this one is shaded hides the answer's
+    // way but leaves the claimed item waiting at the frame's end: the 4K / 2 M
+    // clustered frame took 670 us instead of 590.)
+    uint32_t qi = blockIdx.x;
+    while (qi < qlen) {
         const uint64_t t_start = timed ? clock64() : 0;
         const uint32_t gb = F.queue[qi / PARTS];
         const ViewDev V = F.views[view_of_bin(F, gb)];
@@ -622,6 +626,11 @@ __global__ __launch_bounds__(backend_threads(S, H), backend_min_waves(S, H, STAT
         // a bin's cost is the sum over its strips (zeroed at frame start)
         if (timed && tid == 0)
             atomicAdd((unsigned long long*)&F.bin_cost[gb], (unsigned long long)(clock64() - t_start));
+        if (qlen <= gridDim.x) break;
+        __syncthreads();  // the keys are read
+        if (tid == 0) s_q = gridDim.x + atomicAdd(&F.counters[C_QHEAD], 1u);
+        __syncthreads();
+        qi = s_q;
         __syncthreads();
     }
     if (STATS) {

@@ -228,6 +228,8 @@ struct srg_ctx {
     // and eight kept planes: its grid, which strides over the clip queue, is
     // no larger, so that every workgroup runs in the first round
     uint32_t clip_resident[3] = { 2048, 2048, 2048 };
+    // k_backend workgroups resident per CU, per layout and variant (0: not asked yet)
+    uint32_t backend_resident[8][4] = {};
     hipStream_t stream = nullptr;
     hipStream_t copy_stream = nullptr;  // asynchronous blits
     std::unordered_map<uint64_t, Buffer> buffers;
@@ -638,16 +640,38 @@ bool layout_valid(uint32_t bin_size, uint32_t parts)
     return false;
 }
 
-template <uint32_t S, uint32_t H>
-void launch_backend_t(srg_ctx* ctx, uint32_t wg, bool stats, const FrameDev& F)
+// The back end's workgroups: as many as are resident at once (a workgroup's
+// first item is its own index, so one that had to wait for a place would keep
+// an early, long item waiting: 2,048 workgroups where 1,536 fit took the 4K /
+// 2 M clustered frame from 580 to 645 us), no more than strips.
+template <uint32_t S, uint32_t H, bool STATS, bool WIDE>
+void launch_backend_t(srg_ctx* ctx, uint32_t& resident, const FrameDev& F)
 {
-    const dim3 grid((uint32_t)ctx->num_cus * wg), block(backend_threads(S, H));
+    constexpr uint32_t T = backend_threads(S, H);
+    if (!resident) {
+        int per_cu = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
+                &per_cu, reinterpret_cast<const void*>(&k_backend<S, H, STATS, WIDE>), (int)T, 0) != hipSuccess ||
+            per_cu <= 0) {
+            (void)hipGetLastError();
+            per_cu = 4;
+        }
+        resident = (uint32_t)per_cu;
+    }
+    const uint32_t wg = ctx->cfg.wg_per_cu ? std::min(ctx->cfg.wg_per_cu, resident) : resident;
+    const uint32_t grid = std::min((uint32_t)ctx->num_cus * wg, std::max(1u, F.total_bins * (S / H)));
+    hipLaunchKernelGGL((k_backend<S, H, STATS, WIDE>), dim3(grid), dim3(T), 0, ctx->stream, F);
+}
+
+template <uint32_t S, uint32_t H>
+void launch_backend_t(srg_ctx* ctx, uint32_t resident[4], bool stats, const FrameDev& F)
+{
     if (F.rec_ext) {
-        if (stats) hipLaunchKernelGGL((k_backend<S, H, true, true>), grid, block, 0, ctx->stream, F);
-        else hipLaunchKernelGGL((k_backend<S, H, false, true>), grid, block, 0, ctx->stream, F);
+        if (stats) launch_backend_t<S, H, true, true>(ctx, resident[3], F);
+        else launch_backend_t<S, H, false, true>(ctx, resident[2], F);
     } else {
-        if (stats) hipLaunchKernelGGL((k_backend<S, H, true, false>), grid, block, 0, ctx->stream, F);
-        else hipLaunchKernelGGL((k_backend<S, H, false, false>), grid, block, 0, ctx->stream, F);
+        if (stats) launch_backend_t<S, H, true, false>(ctx, resident[1], F);
+        else launch_backend_t<S, H, false, false>(ctx, resident[0], F);
     }
 }
 
@@ -666,19 +690,17 @@ void launch_setup(srg_ctx* ctx, const FrameDev& F, uint32_t nsingle, uint32_t si
 
 int launch_backend(srg_ctx* ctx, BackendLayout L, const FrameDev& F)
 {
-    // resident workgroups per CU: LDS holds 8 bytes per strip pixel
-    const uint32_t wg = ctx->cfg.wg_per_cu ? ctx->cfg.wg_per_cu
-                      : L.bin_size * L.bin_size / L.parts >= 4096u ? 4u : (L.bin_size == 8 ? 16u : 8u);
     const bool stats = (F.flags & FF_STATS) != 0;
+    uint32_t(*r)[4] = ctx->backend_resident;
     switch (L.bin_size * 8u + L.parts) {
-    case 8 * 8 + 1: launch_backend_t<8, 8>(ctx, wg, stats, F); break;
-    case 16 * 8 + 1: launch_backend_t<16, 16>(ctx, wg, stats, F); break;
-    case 32 * 8 + 1: launch_backend_t<32, 32>(ctx, wg, stats, F); break;
-    case 32 * 8 + 2: launch_backend_t<32, 16>(ctx, wg, stats, F); break;
-    case 32 * 8 + 4: launch_backend_t<32, 8>(ctx, wg, stats, F); break;
-    case 64 * 8 + 1: launch_backend_t<64, 64>(ctx, wg, stats, F); break;
-    case 64 * 8 + 2: launch_backend_t<64, 32>(ctx, wg, stats, F); break;
-    case 64 * 8 + 4: launch_backend_t<64, 16>(ctx, wg, stats, F); break;
+    case 8 * 8 + 1: launch_backend_t<8, 8>(ctx, r[0], stats, F); break;
+    case 16 * 8 + 1: launch_backend_t<16, 16>(ctx, r[1], stats, F); break;
+    case 32 * 8 + 1: launch_backend_t<32, 32>(ctx, r[2], stats, F); break;
+    case 32 * 8 + 2: launch_backend_t<32, 16>(ctx, r[3], stats, F); break;
+    case 32 * 8 + 4: launch_backend_t<32, 8>(ctx, r[4], stats, F); break;
+    case 64 * 8 + 1: launch_backend_t<64, 64>(ctx, r[5], stats, F); break;
+    case 64 * 8 + 2: launch_backend_t<64, 32>(ctx, r[6], stats, F); break;
+    case 64 * 8 + 4: launch_backend_t<64, 16>(ctx, r[7], stats, F); break;
     default: return SRG_ERR_INVALID;
     }
     return SRG_OK;
