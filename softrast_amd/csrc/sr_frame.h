@@ -139,6 +139,7 @@ struct FrameDev {
     uint32_t* queue;
     uint64_t* bin_cost;    // optional per bin (s_memtime ticks)
     uint32_t* counters;
+    uint4* host_counters;  // host memory for the C_NCOUNTERS counters, written when the scan is done (or null)
     uint32_t flags;
 };
 

@@ -207,14 +207,14 @@ struct BinWalk {
     bool check;
 };
 
-__device__ __forceinline__ BinWalk bin_walk(const ViewDev& V, uint32_t bin_k, uint32_t bin_log2, int32_t xmin,
-                                            int32_t xmax, int32_t ymin, int32_t ymax)
+__device__ __forceinline__ BinWalk bin_walk(uint32_t bins_x, uint32_t bin_base, uint32_t bin_k, uint32_t bin_log2,
+                                            int32_t xmin, int32_t xmax, int32_t ymin, int32_t ymax)
 {
     BinWalk w;
     const uint32_t xlo = (uint32_t)xmin & ~7u, ylo = (uint32_t)ymin & ~7u;
     w.k = bin_k;
-    w.view_bins_x = V.bins_x;
-    w.bin_base = V.bin_base;
+    w.view_bins_x = bins_x;
+    w.bin_base = bin_base;
     w.check = !((((uint32_t)ymax >> 6) - ((uint32_t)ymin >> 6) + 1u) <= 2u);
     if ((uint32_t)xmax <= xlo || (uint32_t)ymax <= ylo) {
         w.sbx0 = w.sby0 = w.nx = w.ncand = 0;
@@ -244,20 +244,21 @@ __device__ __forceinline__ uint32_t reference_tile_entries(const Prim& s)
 // (record, bin) pair with its slot in the (part, bin) list: the count
 // atomic's old value plus the lane's rank among the wave's lanes adding to
 // the same counter. Uniform control flow required; `active` lanes carry a
-// primitive described by (c, dx, dy, bbox) in view V.
+// primitive described by (c, dx, dy, bbox) in the view of bins bin_base,
+// bin_base + 1, ..., bins_x to a row.
 //
 // The wave's (primitive, candidate bin) pairs are compacted: an inclusive
 // prefix of the candidate counts numbers them, and each pass hands 64 of them
 // to the 64 lanes (the owner of pair `it` is the first lane whose prefix
 // exceeds it), so a wave takes ceil(sum / 64) passes rather than as many as
 // its largest primitive has candidates.
-__device__ __forceinline__ void walk_bins(const FrameDev& F, const ViewDev& V, bool active, const int32_t c[3],
+__device__ __forceinline__ void walk_bins(const FrameDev& F, uint32_t bins_x, uint32_t bin_base, bool active, const int32_t c[3],
                                           const int32_t dx[3], const int32_t dy[3], int32_t xmin, int32_t xmax,
                                           int32_t ymin, int32_t ymax, uint32_t rec, uint32_t* ht, bool clip)
 {
     BinWalk w;
     if (active) {
-        w = bin_walk(V, F.bin_k, F.bin_log2, xmin, xmax, ymin, ymax);
+        w = bin_walk(bins_x, bin_base, F.bin_k, F.bin_log2, xmin, xmax, ymin, ymax);
     } else {
         w.sbx0 = w.sby0 = w.nx = w.ncand = 0;
         w.view_bins_x = w.bin_base = 0;
@@ -505,12 +506,19 @@ __global__ __launch_bounds__(kSetupThreads) void k_setup(FrameDev F, const Setup
         }
         // a slot without a primitive is never referenced: nothing is written there
         if (survive) write_record<NS>(F, g, s, d);
-        const uint32_t q = wave_add_amount(&F.counters[C_CLIPQ], clipped ? 1u : 0u);
-        // at most one slot per triangle: never overflows
-        if (clipped) F.clip_queue[q] = make_uint2(g, d);
+        // The clip queue's slots (at most one per triangle: never overflows),
+        // reserved here and filled after the bins are walked, so that the
+        // reservation's round trip overlaps the walk.
+        const unsigned long long cm = __ballot(clipped);
+        uint32_t q = 0;
+        if (cm && lane_id() == 0) q = atomicAdd(&F.counters[C_CLIPQ], (uint32_t)__popcll(cm));
 
         if (stats) block_stats_add(&bs, set_up ? reference_tile_entries(s) : 0u, set_up ? 1u : 0u);
-        walk_bins(F, V, survive, s.c, s.dx, s.dy, s.xmin, s.xmax, s.ymin, s.ymax, g, ht, false);
+        walk_bins(F, V.bins_x, V.bin_base, survive, s.c, s.dx, s.dy, s.xmin, s.xmax, s.ymin, s.ymax, g, ht, false);
+        if (clipped)
+            F.clip_queue[readlane_u32(pin(q), 0) + __builtin_amdgcn_mbcnt_hi((uint32_t)(cm >> 32),
+                                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)cm, 0))] =
+                make_uint2(g, d);
     }
     if (stats) {
         __syncthreads();
@@ -609,12 +617,20 @@ __global__ __launch_bounds__(kClipThreads) void k_clip(FrameDev F)
     for (uint32_t base_i = blockIdx.x * blockDim.x; base_i < n; base_i += stride) {
         const uint32_t qi = base_i + threadIdx.x;
         const bool active = qi < n;
-        uint32_t g = 0, d = 0, nfan = 0, pin = 0;
+        uint32_t g = 0, d = 0, nfan = 0, pin_buf = 0;
+        // what the fan triangles' set-up reads of the draw and its view,
+        // loaded beside the vertices and handed on by shuffles
+        uint32_t wh = 0, nslots = 0, bins_x = 0, bin_base = 0;
         if (active) {
             const uint2 e = F.clip_queue[qi];
             g = e.x;
             d = e.y;
             const DrawDev& D = F.draws[d];
+            const ViewDev& V = F.views[D.view];
+            wh = V.width | (V.height << 16);  // at most 16,384 each
+            nslots = D.nslots;
+            bins_x = V.bins_x;
+            bin_base = V.bin_base;
             float4 v[3];
             float a[3][kWideSlots];
             fetch_triangle<NS>(F, D, g - D.tri_base, v, a);
@@ -626,20 +642,19 @@ __global__ __launch_bounds__(kClipThreads) void k_clip(FrameDev F)
                 poly.at(0, k, 3) = v[k].w;
                 for (uint32_t t = 0; t < NS; ++t) poly.at(0, k, 4 + t) = a[k][t];
             }
-            const uint32_t np = clip_polygon(poly, mor, pin);
+            const uint32_t np = clip_polygon(poly, mor, pin_buf);
             nfan = np >= 3 ? np - 2 : 0;
         }
         __syncthreads();  // polygons are read by other lanes below
-        const uint32_t base = wave_add_amount(&F.counters[C_CLIPREC], nfan);
-        const bool fits = base + nfan <= F.clip_cap;
-        if (nfan && !fits) atomicOr(&F.counters[C_FLAGS], FLAG_CLIP_OVERFLOW);
-        if (nfan && fits) F.clip_base[g] = base;
-        // the wave's fan triangles, one per lane: lane j takes fan item t of
-        // the lane whose inclusive fan count first exceeds t
+        // The wave's fan triangles, one per lane: lane j takes fan item t of
+        // the lane whose inclusive fan count first exceeds t. Their records
+        // take one reservation, whose round trip the first 64's set-up hides.
         const uint32_t lane = lane_id();
-        const uint32_t incl = wave_incl_sum(fits ? nfan : 0u);
+        const uint32_t incl = wave_incl_sum(nfan);
         const uint32_t total = readlane_u32(incl, 63);
-        const uint32_t first = incl - (fits ? nfan : 0u);
+        const uint32_t first = incl - nfan;
+        uint32_t reserved = 0;
+        if (lane == 0 && total) reserved = atomicAdd(&F.counters[C_CLIPREC], total);
         for (uint32_t t0 = 0; t0 < total; t0 += 64) {
             const uint32_t t = t0 + lane;
             uint32_t lo = 0, hi = 63;
@@ -650,13 +665,12 @@ __global__ __launch_bounds__(kClipThreads) void k_clip(FrameDev F)
                 else lo = mid + 1;
             }
             const int src = (int)(t < total ? lo : 0u);
-            const uint32_t og = __shfl(g, src, 64), od = __shfl(d, src, 64), opin = __shfl(pin, src, 64);
-            const uint32_t obase = __shfl(base, src, 64), j = t - __shfl(first, src, 64);
-            const DrawDev& D = F.draws[od];
-            const ViewDev& V = F.views[D.view];
+            const uint32_t og = __shfl(g, src, 64), od = __shfl(d, src, 64), opin = __shfl(pin_buf, src, 64);
+            const uint32_t ofirst = __shfl(first, src, 64), onfan = __shfl(nfan, src, 64), j = t - ofirst;
+            const uint32_t owh = __shfl(wh, src, 64), onslots = __shfl(nslots, src, 64);
+            const uint32_t obx = __shfl(bins_x, src, 64), obb = __shfl(bin_base, src, 64);
             Prim s;
             bool ok = false;
-            uint32_t r = 0;
             if (t < total) {
                 const ClipPoly<NS> owner{ poly.lds, (uint32_t)src };
                 const float4 fv[3] = { owner.pos(opin, 0), owner.pos(opin, j + 1), owner.pos(opin, j + 2) };
@@ -666,12 +680,18 @@ __global__ __launch_bounds__(kClipThreads) void k_clip(FrameDev F)
                     fa[1][a] = owner.at(opin, j + 1, 4 + a);
                     fa[2][a] = owner.at(opin, j + 2, 4 + a);
                 }
-                r = F.ntris + obase + j;
-                ok = setup_prim<NS>(s, fv, fa, D.nslots, V.width, V.height);
-                if (ok) {
-                    write_record<NS>(F, r, s, od);
-                    F.clip_order[obase + j] = (og << 3) | j;
-                }
+                ok = setup_prim<NS>(s, fv, fa, onslots, owh & 0xFFFFu, owh >> 16);
+            }
+            const uint32_t obase = readlane_u32(pin(reserved), 0) + ofirst;
+            // a triangle whose records do not fit keeps none of them: the frame is rendered again
+            const bool fits = obase + onfan <= F.clip_cap;
+            if (t < total && !fits) atomicOr(&F.counters[C_FLAGS], FLAG_CLIP_OVERFLOW);
+            const uint32_t r = F.ntris + obase + j;
+            ok = ok && fits;
+            if (t < total && fits && j == 0) F.clip_base[og] = obase;
+            if (ok) {
+                write_record<NS>(F, r, s, od);
+                F.clip_order[obase + j] = (og << 3) | j;
             }
             if (F.flags & FF_STATS) {
                 const uint32_t te = wave_sum(ok ? reference_tile_entries(s) : 0u);
@@ -679,7 +699,7 @@ __global__ __launch_bounds__(kClipThreads) void k_clip(FrameDev F)
                 if (lane == 0 && te) atomicAdd(&F.counters[C_TILE_ENTRIES], te);
                 if (lane == 0 && pr) atomicAdd(&F.counters[C_PRIMS], pr);
             }
-            walk_bins(F, V, ok, s.c, s.dx, s.dy, s.xmin, s.xmax, s.ymin, s.ymax, r, ht, true);
+            walk_bins(F, obx, obb, ok, s.c, s.dx, s.dy, s.xmin, s.xmax, s.ymin, s.ymax, r, ht, true);
         }
         __syncthreads();  // before the polygons are overwritten
     }
@@ -764,15 +784,30 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_blocks(FrameDev F, uint32
 
 // The frame totals: entries (the end of the last bin's list) and queue
 // length, the entry arena's overflow check and the clip regions' pair count.
+// The counters of the kernels before are final here, so this is also where
+// the host gets them.
 __device__ __forceinline__ void scan_totals(const FrameDev& F, uint32_t tc, uint32_t tq)
 {
     F.bin_start[F.total_bins] = tc;
     F.counters[C_ENTRIES] = tc;
     F.counters[C_QLEN] = tq;
-    if (tc > F.entry_cap) atomicOr(&F.counters[C_FLAGS], FLAG_ENTRY_OVERFLOW);
+    const bool overflow = tc > F.entry_cap;
+    if (overflow) atomicOr(&F.counters[C_FLAGS], FLAG_ENTRY_OVERFLOW);
     uint32_t cp = 0;
     for (uint32_t i = 0; i < kClipPairRegions; ++i) cp += F.pair_count[(F.pair_regions + i) * kPairStride];
     F.counters[C_CLIP_PAIRS] = cp;
+    if (F.host_counters) {
+        uint32_t c[C_NCOUNTERS];
+#pragma unroll
+        for (uint32_t i = 0; i < C_NCOUNTERS; ++i) c[i] = F.counters[i];
+        c[C_ENTRIES] = tc;
+        c[C_QLEN] = tq;
+        c[C_CLIP_PAIRS] = cp;
+        c[C_FLAGS] |= overflow ? FLAG_ENTRY_OVERFLOW : 0u;
+        static_assert(C_NCOUNTERS == 16, "four 16-byte words");
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) F.host_counters[i] = make_uint4(c[4 * i], c[4 * i + 1], c[4 * i + 2], c[4 * i + 3]);
+    }
 }
 
 // Pass 2 (one workgroup): block offsets and the frame totals.

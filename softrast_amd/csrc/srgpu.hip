@@ -14,6 +14,7 @@
 // in-order strict reverse-Z test followed by in-order shading leaves in the
 // pixel, so bin entries may arrive in any order.
 #include <hip/hip_runtime.h>
+#include <hip/hip_ext.h>
 
 #include <algorithm>
 #include <atomic>
@@ -52,16 +53,20 @@ static uint64_t clip_pair_want(uint32_t clip_pairs)
     return (uint64_t)clip_pairs * 2 * kClipPairRegions * 5 / 4;
 }
 
-__global__ void k_frame_init(uint32_t* counters, uint32_t* part_count, uint64_t* bin_cost, uint32_t nbins,
-                             uint32_t* gate, uint32_t every)
+// The frame's tables come along: `ntab` 16-byte words read from page-locked
+// host memory (a copy of their own is a launch more, about 3 us a frame).
+__global__ __launch_bounds__(256) void k_frame_init(uint32_t* counters, uint32_t* part_count, uint64_t* bin_cost,
+                                                    uint32_t nbins, uint32_t* gate, uint32_t every, const uint4* htab,
+                                                    uint4* tab, uint32_t ntab)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x, n = gridDim.x * blockDim.x;
     if (gate && i == 0) {
         gate[1] = (every <= 1u || gate[0] % every == 0u) ? 1u : 0u;
         gate[0] = gate[0] + 1u;
     }
-    for (uint32_t t = i; t < kCounterWords; t += gridDim.x * blockDim.x) counters[t] = 0;
-    for (uint32_t t = i; t < nbins * kBinParts; t += gridDim.x * blockDim.x) {
+    for (uint32_t t = i; t < ntab; t += n) tab[t] = htab[t];
+    for (uint32_t t = i; t < kCounterWords; t += n) counters[t] = 0;
+    for (uint32_t t = i; t < nbins * kBinParts; t += n) {
         part_count[t] = 0;
         if (t < nbins) bin_cost[t] = 0;
     }
@@ -258,6 +263,7 @@ struct srg_ctx {
     DevArray<uint32_t> blit_staging;    // rows for a blit to memory that is neither host allocation nor page-locked
     uint32_t* stage = nullptr;          // two page-locked chunks through which pageable memory is written (staged_out)
     hipEvent_t stage_ev[2] = {};
+    hipEvent_t done = nullptr;          // recorded by a frame's or a blit's last kernel
     DevArray<uint8_t> tex_work;         // texture building: base image, filtered rows, weights
     uint32_t* h_counters = nullptr;
     uint32_t clip_cap = 0, entry_cap = 0;
@@ -375,14 +381,18 @@ void blit_host_fn(void* arg)
 // the compute units to the frame that renders meanwhile.
 constexpr uint32_t kAsyncBlitBlocks = 64;
 
+// stop: an event that the kernel records (or null).
 void launch_detile(hipStream_t stream, uint32_t max_blocks, const uint32_t* tiles, uint32_t* out, const srg_fb* fb,
-                   uint32_t y0, uint32_t rows, bool bgra)
+                   uint32_t y0, uint32_t rows, bool bgra, hipEvent_t stop)
 {
     const dim3 grid(std::min(rows, max_blocks)), block(256);
+    const uint32_t swap = bgra ? 1u : 0u;
     if (fb->width % 4 == 0 && ((uintptr_t)out & 15u) == 0)
-        hipLaunchKernelGGL(k_detile<4>, grid, block, 0, stream, tiles, out, fb->width, y0, rows, fb->tiles_x, bgra ? 1u : 0u);
+        hipExtLaunchKernelGGL(k_detile<4>, grid, block, 0, stream, nullptr, stop, 0, tiles, out, fb->width, y0, rows,
+                              fb->tiles_x, swap);
     else
-        hipLaunchKernelGGL(k_detile<1>, grid, block, 0, stream, tiles, out, fb->width, y0, rows, fb->tiles_x, bgra ? 1u : 0u);
+        hipExtLaunchKernelGGL(k_detile<1>, grid, block, 0, stream, nullptr, stop, 0, tiles, out, fb->width, y0, rows,
+                              fb->tiles_x, swap);
 }
 
 // Where results for the caller's memory [p, p + bytes) are written.
@@ -415,9 +425,9 @@ HostDst classify_dst(void* p, size_t bytes, uint32_t** dev)
 }
 
 // Writes `units` pieces of unit_bytes (at most kStageBytes) each to pageable
-// memory at dst: emit(out, first, n) launches on the library stream the
+// memory at dst: emit(out, first, n, stop) launches on the library stream the
 // kernel that writes pieces first .. first + n - 1 to page-locked memory at
-// out; the host copies one chunk to dst while the next is written. A chunk of
+// out and records stop; the host copies one chunk to dst while the next is written. A chunk of
 // 512 KiB takes 9 us on the link and 17 us to copy on, so the link is hidden
 // but for the first chunk. Measured with the same bytes through the runtime's
 // copy of a device staging buffer: 230 KB 21 against 44 us, 8.3 MB 425 (with
@@ -429,16 +439,14 @@ int staged_out(srg_ctx* ctx, void* dst, size_t units, size_t unit_bytes, Emit em
     auto start = [&](size_t c) -> int {
         uint32_t* out = nullptr;
         HIP_TRY(hipHostGetDevicePointer((void**)&out, ctx->stage + (c & 1) * (kStageBytes / 4), 0));
-        emit(out, c * per, std::min(per, units - c * per));
+        emit(out, c * per, std::min(per, units - c * per), ctx->stage_ev[c & 1]);
         HIP_TRY(hipGetLastError());
-        if (nchunks > 1) HIP_TRY(hipEventRecord(ctx->stage_ev[c & 1], ctx->stream));
         return SRG_OK;
     };
     int st = SRG_OK;
     for (size_t c = 0; c < std::min<size_t>(2, nchunks) && !st; ++c) st = start(c);
     for (size_t c = 0; c < nchunks && !st; ++c) {
-        if ((nchunks > 1 ? hipEventSynchronize(ctx->stage_ev[c & 1]) : hipStreamSynchronize(ctx->stream)) != hipSuccess)
-            return SRG_ERR_HIP;
+        HIP_TRY(hipEventSynchronize(ctx->stage_ev[c & 1]));
         std::memcpy((uint8_t*)dst + c * per * unit_bytes, ctx->stage + (c & 1) * (kStageBytes / 4),
                     std::min(per, units - c * per) * unit_bytes);
         if (c + 2 < nchunks) st = start(c + 2);
@@ -459,12 +467,14 @@ int copy_out(srg_ctx* ctx, void* dst, const uint32_t* src, size_t words)
     }
     constexpr size_t unit = 1024;  // words
     const size_t whole = words / unit;
-    int st = staged_out(ctx, dst, whole, unit * 4, [&](uint32_t* out, size_t first, size_t n) {
-        hipLaunchKernelGGL(k_copy_out, dim3((uint32_t)n), dim3(256), 0, ctx->stream, src + first * unit, out, n * unit);
+    int st = staged_out(ctx, dst, whole, unit * 4, [&](uint32_t* out, size_t first, size_t n, hipEvent_t stop) {
+        hipExtLaunchKernelGGL(k_copy_out, dim3((uint32_t)n), dim3(256), 0, ctx->stream, nullptr, stop, 0, src + first * unit,
+                              out, n * unit);
     });
     if (!st && words % unit)
-        st = staged_out(ctx, (uint32_t*)dst + whole * unit, 1, (words % unit) * 4, [&](uint32_t* out, size_t, size_t) {
-            hipLaunchKernelGGL(k_copy_out, dim3(4), dim3(256), 0, ctx->stream, src + whole * unit, out, words % unit);
+        st = staged_out(ctx, (uint32_t*)dst + whole * unit, 1, (words % unit) * 4, [&](uint32_t* out, size_t, size_t, hipEvent_t stop) {
+            hipExtLaunchKernelGGL(k_copy_out, dim3(4), dim3(256), 0, ctx->stream, nullptr, stop, 0, src + whole * unit, out,
+                                  words % unit);
         });
     return st;
 }
@@ -645,7 +655,7 @@ bool layout_valid(uint32_t bin_size, uint32_t parts)
 // an early, long item waiting: 2,048 workgroups where 1,536 fit took the 4K /
 // 2 M clustered frame from 580 to 645 us), no more than strips.
 template <uint32_t S, uint32_t H, bool STATS, bool WIDE>
-void launch_backend_t(srg_ctx* ctx, uint32_t& resident, const FrameDev& F)
+void launch_backend_t(srg_ctx* ctx, uint32_t& resident, const FrameDev& F, hipEvent_t stop)
 {
     constexpr uint32_t T = backend_threads(S, H);
     if (!resident) {
@@ -660,18 +670,21 @@ void launch_backend_t(srg_ctx* ctx, uint32_t& resident, const FrameDev& F)
     }
     const uint32_t wg = ctx->cfg.wg_per_cu ? std::min(ctx->cfg.wg_per_cu, resident) : resident;
     const uint32_t grid = std::min((uint32_t)ctx->num_cus * wg, std::max(1u, F.total_bins * (S / H)));
-    hipLaunchKernelGGL((k_backend<S, H, STATS, WIDE>), dim3(grid), dim3(T), 0, ctx->stream, F);
+    if (stop)
+        hipExtLaunchKernelGGL((k_backend<S, H, STATS, WIDE>), dim3(grid), dim3(T), 0, ctx->stream, nullptr, stop, 0, F);
+    else
+        hipLaunchKernelGGL((k_backend<S, H, STATS, WIDE>), dim3(grid), dim3(T), 0, ctx->stream, F);
 }
 
 template <uint32_t S, uint32_t H>
-void launch_backend_t(srg_ctx* ctx, uint32_t resident[4], bool stats, const FrameDev& F)
+void launch_backend_t(srg_ctx* ctx, uint32_t resident[4], bool stats, const FrameDev& F, hipEvent_t stop)
 {
     if (F.rec_ext) {
-        if (stats) launch_backend_t<S, H, true, true>(ctx, resident[3], F);
-        else launch_backend_t<S, H, false, true>(ctx, resident[2], F);
+        if (stats) launch_backend_t<S, H, true, true>(ctx, resident[3], F, stop);
+        else launch_backend_t<S, H, false, true>(ctx, resident[2], F, stop);
     } else {
-        if (stats) launch_backend_t<S, H, true, false>(ctx, resident[1], F);
-        else launch_backend_t<S, H, false, false>(ctx, resident[0], F);
+        if (stats) launch_backend_t<S, H, true, false>(ctx, resident[1], F, stop);
+        else launch_backend_t<S, H, false, false>(ctx, resident[0], F, stop);
     }
 }
 
@@ -688,19 +701,19 @@ void launch_setup(srg_ctx* ctx, const FrameDev& F, uint32_t nsingle, uint32_t si
                            F, F.groups, F.group_members, F.draws, F.views, nsingle, F.ngroups, single_blocks);
 }
 
-int launch_backend(srg_ctx* ctx, BackendLayout L, const FrameDev& F)
+int launch_backend(srg_ctx* ctx, BackendLayout L, const FrameDev& F, hipEvent_t stop)
 {
     const bool stats = (F.flags & FF_STATS) != 0;
     uint32_t(*r)[4] = ctx->backend_resident;
     switch (L.bin_size * 8u + L.parts) {
-    case 8 * 8 + 1: launch_backend_t<8, 8>(ctx, r[0], stats, F); break;
-    case 16 * 8 + 1: launch_backend_t<16, 16>(ctx, r[1], stats, F); break;
-    case 32 * 8 + 1: launch_backend_t<32, 32>(ctx, r[2], stats, F); break;
-    case 32 * 8 + 2: launch_backend_t<32, 16>(ctx, r[3], stats, F); break;
-    case 32 * 8 + 4: launch_backend_t<32, 8>(ctx, r[4], stats, F); break;
-    case 64 * 8 + 1: launch_backend_t<64, 64>(ctx, r[5], stats, F); break;
-    case 64 * 8 + 2: launch_backend_t<64, 32>(ctx, r[6], stats, F); break;
-    case 64 * 8 + 4: launch_backend_t<64, 16>(ctx, r[7], stats, F); break;
+    case 8 * 8 + 1: launch_backend_t<8, 8>(ctx, r[0], stats, F, stop); break;
+    case 16 * 8 + 1: launch_backend_t<16, 16>(ctx, r[1], stats, F, stop); break;
+    case 32 * 8 + 1: launch_backend_t<32, 32>(ctx, r[2], stats, F, stop); break;
+    case 32 * 8 + 2: launch_backend_t<32, 16>(ctx, r[3], stats, F, stop); break;
+    case 32 * 8 + 4: launch_backend_t<32, 8>(ctx, r[4], stats, F, stop); break;
+    case 64 * 8 + 1: launch_backend_t<64, 64>(ctx, r[5], stats, F, stop); break;
+    case 64 * 8 + 2: launch_backend_t<64, 32>(ctx, r[6], stats, F, stop); break;
+    case 64 * 8 + 4: launch_backend_t<64, 16>(ctx, r[7], stats, F, stop); break;
     default: return SRG_ERR_INVALID;
     }
     return SRG_OK;
@@ -1133,7 +1146,8 @@ int run_frame(srg_ctx* ctx, bool noalloc)
             std::max<uint32_t>(1, std::min<uint32_t>((F.pair_region_cap + emit_chunk - 1) / emit_chunk, 4096));
         const uint32_t clip_blocks = std::max<uint32_t>(
             1, std::min<uint32_t>((NT + kClipThreads - 1) / kClipThreads, ctx->clip_resident[wide ? 2 : (narrow ? 0 : 1)]));
-        const uint32_t init_blocks = std::max<uint32_t>(1, std::min<uint32_t>((kBinParts * TB + 255) / 256, 1024));
+        const uint32_t init_blocks = std::min<uint32_t>(
+            std::max<uint32_t>((kBinParts * TB + 255) / 256, (uint32_t)(off / 16 + 255) / 256), 1024);
         const uint32_t scan_blocks = (TB + kScanThreads - 1) / kScanThreads;
         const bool ordered = ctx->cfg.tile_order != SRG_ORDER_NATURAL;
         // while the autotuner sweeps, the learned order falls back to entry
@@ -1171,12 +1185,21 @@ int run_frame(srg_ctx* ctx, bool noalloc)
             hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, ctx->stream, ctx->sched_gate, 0u, (size_t)1);
             HIP_TRY(hipGetLastError());
         }
+        // The frame's counters are final after the scan, which then writes
+        // them to the host itself, unless the back end counts fragments
+        // (statistics) or the learned order records after it. (A copy of
+        // their own after the back end costs about 4 us.)
+        const bool late_counters = (F.flags & FF_STATS) || learned;
+        void *h_tables_dev = nullptr, *h_counters_dev = nullptr;
+        HIP_TRY(hipHostGetDevicePointer(&h_tables_dev, ctx->h_tables, 0));
+        HIP_TRY(hipHostGetDevicePointer(&h_counters_dev, ctx->h_counters, 0));
+        F.host_counters = late_counters ? nullptr : (uint4*)h_counters_dev;
         // The whole frame on the stream: tables, six kernels, counters back.
-        auto enqueue = [&](bool split_events) -> int {
-            HIP_TRY(hipMemcpyAsync(A.tables, ctx->h_tables, off, hipMemcpyHostToDevice, ctx->stream));
+        // stop: recorded by the last kernel (a back end without late counters), or null.
+        auto enqueue = [&](bool split_events, hipEvent_t stop) -> int {
             hipLaunchKernelGGL(k_frame_init, dim3(init_blocks), dim3(256), 0, ctx->stream, A.counters,
-                               A.part_count, A.bin_cost, TB,
-                               learned ? ctx->sched_gate : nullptr, sched_every);
+                               A.part_count, A.bin_cost, TB, learned ? ctx->sched_gate : nullptr, sched_every,
+                               (const uint4*)h_tables_dev, (uint4*)A.tables, (uint32_t)(off / 16));
             if (ctx->cfg.flags & SRG_CFG_KEEP_PRIMID)
                 for (auto& v : vdev)
                     if (v.primid)
@@ -1223,7 +1246,7 @@ int run_frame(srg_ctx* ctx, bool noalloc)
                                    (const uint32_t*)A.order_hist);
             }
             if (split_events) HIP_TRY(hipEventRecord(ctx->ev[1], ctx->stream));
-            if (const int lst = launch_backend(ctx, L, F)) return lst;
+            if (const int lst = launch_backend(ctx, L, F, stop)) return lst;
             if (split_events) HIP_TRY(hipEventRecord(ctx->ev[4], ctx->stream));
             if (learned)
                 hipLaunchKernelGGL(k_mlp_record, dim3((TB + 255) / 256), dim3(256), 0, ctx->stream, F,
@@ -1231,13 +1254,14 @@ int run_frame(srg_ctx* ctx, bool noalloc)
                                    (const float*)(ctx->sched_trained ? ctx->sched_pred.ptr : nullptr), ctx->sched_ring,
                                    kSchedRing, ctx->sched_head);
             HIP_TRY(hipGetLastError());
-            HIP_TRY(hipMemcpyAsync(ctx->h_counters, A.counters, sizeof(uint32_t) * C_NCOUNTERS,
-                                   hipMemcpyDeviceToHost, ctx->stream));
+            if (late_counters)
+                HIP_TRY(hipMemcpyAsync(ctx->h_counters, A.counters, sizeof(uint32_t) * C_NCOUNTERS,
+                                       hipMemcpyDeviceToHost, ctx->stream));
             return SRG_OK;
         };
 
         const bool timing = (ctx->cfg.flags & SRG_CFG_TIMING) != 0 || sweeping;
-        bool split = false;
+        bool split = false, own_stop = false;
         if ((ctx->cfg.flags & SRG_CFG_GRAPH) && !noalloc) {
             // Replay the captured frame when nothing it depends on changed:
             // the table bytes, every pointer and capacity in F, and the
@@ -1256,7 +1280,7 @@ int run_frame(srg_ctx* ctx, bool noalloc)
                 ctx->graph_exec = nullptr;
                 hipGraph_t graph = nullptr;
                 HIP_TRY(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-                const int est = enqueue(false);
+                const int est = enqueue(false, nullptr);
                 const hipError_t cerr = hipStreamEndCapture(ctx->stream, &graph);
                 if (est) return est;
                 if (cerr != hipSuccess) return SRG_ERR_HIP;
@@ -1274,11 +1298,14 @@ int run_frame(srg_ctx* ctx, bool noalloc)
             if (timing) HIP_TRY(hipEventRecord(ctx->ev[2], ctx->stream));
         } else {
             if (timing) HIP_TRY(hipEventRecord(ctx->ev[0], ctx->stream));
-            if ((st = enqueue(timing))) return st;
+            own_stop = !timing && !late_counters;
+            if ((st = enqueue(timing, own_stop ? ctx->done : nullptr))) return st;
             if (timing) HIP_TRY(hipEventRecord(ctx->ev[2], ctx->stream));
             split = timing;
         }
-        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        // waiting for an event of the last kernel itself returns 2.7 us before
+        // a stream synchronisation, which adds a packet of its own
+        HIP_TRY(own_stop ? hipEventSynchronize(ctx->done) : hipStreamSynchronize(ctx->stream));
 
         const uint32_t flags = ctx->h_counters[C_FLAGS];
         if (flags & FLAG_INDEX_RANGE) return SRG_ERR_INDEX_RANGE;
@@ -1425,8 +1452,8 @@ int srg_create(const srg_config* cfg, srg_ctx** out)
     }
     for (auto& e : ctx->ev)
         if (hipEventCreate(&e) != hipSuccess) { srg_destroy(ctx); return SRG_ERR_HIP; }
-    for (auto& e : ctx->stage_ev)
-        if (hipEventCreateWithFlags(&e, hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess) {
+    for (hipEvent_t* e : { &ctx->stage_ev[0], &ctx->stage_ev[1], &ctx->done })
+        if (hipEventCreateWithFlags(e, hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess) {
             srg_destroy(ctx);
             return SRG_ERR_HIP;
         }
@@ -1487,7 +1514,7 @@ void srg_destroy(srg_ctx* ctx)
     if (ctx->h_tables) (void)hipHostFree(ctx->h_tables);
     if (ctx->h_counters) (void)hipHostFree(ctx->h_counters);
     if (ctx->stage) (void)hipHostFree(ctx->stage);
-    for (auto& e : ctx->stage_ev)
+    for (hipEvent_t e : { ctx->stage_ev[0], ctx->stage_ev[1], ctx->done })
         if (e) (void)hipEventDestroy(e);
     for (auto& e : ctx->ev)
         if (e) (void)hipEventDestroy(e);
@@ -1788,24 +1815,30 @@ int srg_blit(srg_ctx* ctx, srg_fb* fb, void* linear, void (*on_finish)(void*), v
     int st = flush_pending_clear(ctx, fb, fb->write_plane);
     if (st) return st;
     const size_t npx = (size_t)fb->width * fb->height;
-    auto detile = [&](uint32_t* out, uint32_t y0, uint32_t rows) {
-        launch_detile(ctx->stream, 256, p.colour, out, fb, y0, rows, false);
+    auto detile = [&](uint32_t* out, uint32_t y0, uint32_t rows, hipEvent_t stop) {
+        launch_detile(ctx->stream, 256, p.colour, out, fb, y0, rows, false, stop);
     };
     uint32_t* dst = nullptr;
     const HostDst kind = classify_dst(linear, npx * 4, &dst);
     if (kind == HostDst::pageable) {
         st = staged_out(ctx, linear, fb->height, (size_t)fb->width * 4,
-                        [&](uint32_t* out, size_t first, size_t n) { detile(out, (uint32_t)first, (uint32_t)n); });
+                        [&](uint32_t* out, size_t first, size_t n, hipEvent_t stop) {
+                            detile(out, (uint32_t)first, (uint32_t)n, stop);
+                        });
         if (st) return st;
     } else {
         if (kind == HostDst::other) {
             if ((st = ctx->blit_staging.ensure(npx))) return st;
             dst = ctx->blit_staging.ptr;
         }
-        detile(dst, 0, fb->height);
+        detile(dst, 0, fb->height, ctx->done);
         HIP_TRY(hipGetLastError());
-        if (kind == HostDst::other) HIP_TRY(hipMemcpyAsync(linear, dst, npx * 4, hipMemcpyDeviceToHost, ctx->stream));
-        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        if (kind == HostDst::other) {
+            HIP_TRY(hipMemcpyAsync(linear, dst, npx * 4, hipMemcpyDeviceToHost, ctx->stream));
+            HIP_TRY(hipStreamSynchronize(ctx->stream));
+        } else {
+            HIP_TRY(hipEventSynchronize(ctx->done));
+        }
     }
     fb->write_plane ^= 1u;
     if (on_finish) on_finish(user);
@@ -1837,7 +1870,8 @@ int srg_blit_async(srg_ctx* ctx, srg_fb* fb, void* linear, uint32_t flags, void 
     // the copy stream starts once the frame that wrote the plane is done
     HIP_TRY(hipEventRecord(ctx->ev[3], ctx->stream));
     HIP_TRY(hipStreamWaitEvent(ctx->copy_stream, ctx->ev[3], 0));
-    launch_detile(ctx->copy_stream, kAsyncBlitBlocks, p.colour, dst, fb, 0, fb->height, (flags & SRG_BLIT_BGRA) != 0);
+    launch_detile(ctx->copy_stream, kAsyncBlitBlocks, p.colour, dst, fb, 0, fb->height, (flags & SRG_BLIT_BGRA) != 0,
+                  nullptr);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(p.read_done, ctx->copy_stream));
     p.job = BlitJob{ linear, direct ? nullptr : p.pinned, npx * 4, on_finish, user };
