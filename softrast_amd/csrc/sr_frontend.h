@@ -240,6 +240,69 @@ __device__ __forceinline__ uint32_t reference_tile_entries(const Prim& s)
     return n;
 }
 
+// i / nx and i % nx for a primitive's candidate i (i < nx * ny <= 2^22, so
+// i / nx < 2^11): the quotient from the fp32 reciprocal is within 2^-11 of
+// i / nx, so its truncation is off by at most one, which one correction step
+// fixes.
+__device__ __forceinline__ void cand_xy(uint32_t i, uint32_t nx, uint32_t& x, uint32_t& y)
+{
+    uint32_t q = (uint32_t)((float)i * __builtin_amdgcn_rcpf((float)nx));
+    int32_t r = (int32_t)(i - __umul24(q, nx));
+    if (r < 0) {
+        q -= 1u;
+        r += (int32_t)nx;
+    } else if (r >= (int32_t)nx) {
+        q += 1u;
+        r -= (int32_t)nx;
+    }
+    x = (uint32_t)r;
+    y = q;
+}
+
+// The bins of one primitive of n candidates, every argument the same in all
+// lanes: 64 candidates a step, four steps' count atomics in flight. Its pairs
+// go to slots at, at + 1, ... of the region at first_p. Through the compacted
+// passes one wave with a few screen-covering triangles took 100 us of k_clip's
+// 122 on 24 mixed views; now k_clip takes 56 there and 27 instead of 39 at
+// 960x540 inside the geometry. From 32 or 16 candidates on instead of 64, both
+// stay as they are and k_setup<8> takes 32.7 or 39.2 us instead of 29.5 (1080p
+// / 250 k).
+constexpr uint32_t kBigCand = 64;
+__device__ __forceinline__ void walk_big(const FrameDev& F, uint32_t n, uint32_t org, uint32_t pn, uint32_t bins_x,
+                                         uint32_t bin_base, uint32_t rec, const int32_t c[3], const int32_t dx[3],
+                                         const int32_t dy[3], uint32_t first_p, uint32_t at, uint32_t cap)
+{
+    const uint32_t nx = pn & 0x7FFFFFFFu, part = part_of(rec) * F.total_bins;
+    const bool check = (pn >> 31) != 0;
+    for (uint32_t base = 0; base < n; base += 256) {
+        uint32_t key[4], slot[4];
+        bool act[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t i = base + 64u * k + lane_id();
+            uint32_t x, y;
+            cand_xy(i, nx, x, y);
+            x += org & 0xFFFFu;
+            y += org >> 16;
+            act[k] = i < n && (!check || tile_accepts(c, dx, dy, (x >> F.bin_klog2) * kBin, (y >> F.bin_klog2) * kBin));
+            key[k] = part + bin_base + y * bins_x + x;
+            slot[k] = 0;
+            if (act[k]) slot[k] = atomicAdd(&F.part_count[key[k]], 1u);
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t i = base + 64u * k + lane_id(), p = first_p + at + i, np = F.pair_total;
+            if (i < n && at + i < cap) {
+                F.pairs[p] = act[k] ? rec : kNoPair;
+                if (act[k]) {
+                    F.pairs[np + p] = key[k];
+                    F.pairs[2u * np + p] = slot[k];
+                }
+            }
+        }
+    }
+}
+
 // Counts a primitive's bin entries, wave-aggregated, and records each
 // (record, bin) pair with its slot in the (part, bin) list: the count
 // atomic's old value plus the lane's rank among the wave's lanes adding to
@@ -251,7 +314,10 @@ __device__ __forceinline__ uint32_t reference_tile_entries(const Prim& s)
 // prefix of the candidate counts numbers them, and each pass hands 64 of them
 // to the 64 lanes (the owner of pair `it` is the first lane whose prefix
 // exceeds it), so a wave takes ceil(sum / 64) passes rather than as many as
-// its largest primitive has candidates.
+// its largest primitive has candidates. A primitive with kBigCand candidates
+// or more is walked by itself, 64 candidates a step (walk_big): its passes are
+// full without compaction and its bins all different, so they need neither the
+// owner search nor the hash.
 __device__ __forceinline__ void walk_bins(const FrameDev& F, uint32_t bins_x, uint32_t bin_base, bool active, const int32_t c[3],
                                           const int32_t dx[3], const int32_t dy[3], int32_t xmin, int32_t xmax,
                                           int32_t ymin, int32_t ymax, uint32_t rec, uint32_t* ht, bool clip)
@@ -265,12 +331,16 @@ __device__ __forceinline__ void walk_bins(const FrameDev& F, uint32_t bins_x, ui
         w.check = false;
     }
     const uint32_t lane = lane_id();
-    const uint32_t incl = wave_incl_sum(w.ncand);
+    unsigned long long bigs = __ballot(w.ncand >= kBigCand);
+    const uint32_t ncand = w.ncand >= kBigCand ? 0u : w.ncand;
+    const uint32_t incl = wave_incl_sum(ncand);
     const uint32_t total = readlane_u32(incl, 63);
-    const uint32_t first = incl - w.ncand;
+    const uint32_t first = incl - ncand;
+    uint32_t total_all = total;
+    if (bigs) total_all += readlane_u32(wave_incl_sum(w.ncand - ncand), 63);
     const uint32_t pk_org = w.sbx0 | (w.sby0 << 16);                  // bin coordinates < 2^16
     const uint32_t pk_nx = max(w.nx, 1u) | ((w.check ? 1u : 0u) << 31);  // nx < 2^31
-    const bool any_check = __ballot(w.check && w.ncand != 0) != 0ull;
+    const bool any_check = __ballot(w.check && ncand != 0) != 0ull;
     // The wave's pairs take one reservation in its region, issued before the
     // passes so that its round trip overlaps their work: candidate `it` goes
     // to slot pbase + it, and one the corner test rejects leaves a hole
@@ -281,31 +351,22 @@ __device__ __forceinline__ void walk_bins(const FrameDev& F, uint32_t bins_x, ui
     const uint32_t first_p = clip ? F.pair_regions * F.pair_region_cap + (region - F.pair_regions) * F.clip_pair_cap
                                   : region * F.pair_region_cap;
     uint32_t pres = 0;
-    if (lane == 0 && total) pres = atomicAdd(&F.pair_count[region * kPairStride], total);
+    if (lane == 0 && total_all) pres = atomicAdd(&F.pair_count[region * kPairStride], total_all);
     uint32_t carry = 0;
     for (uint32_t base = 0; base < total; base += 64) {
         const uint32_t it = base + lane;
         const bool valid = it < total;
-        const uint32_t m = wave_owner(ht + kHashWords, w.ncand, first, base, carry);
+        const uint32_t m = wave_owner(ht + kHashWords, ncand, first, base, carry);
         const int src = (int)(valid && m ? min(m - 1u, 63u) : 0u);
         const uint32_t org = __shfl(pk_org, src, 64), pn = __shfl(pk_nx, src, 64);
         const uint32_t i = it - __shfl(first, src, 64);
         const uint32_t bb = __shfl(w.bin_base, src, 64), vbx = __shfl(w.view_bins_x, src, 64);
         const uint32_t orec = __shfl(rec, src, 64);
         const uint32_t nx = pn & 0x7FFFFFFFu;
-        // i / nx and i % nx (i < nx * ny <= 2^22, so i / nx < 2^11): the
-        // quotient from the fp32 reciprocal is within 2^-11 of i / nx, so its
-        // truncation is off by at most one, which one correction step fixes
-        uint32_t q = (uint32_t)((float)i * __builtin_amdgcn_rcpf((float)nx));
-        int32_t r = (int32_t)(i - __umul24(q, nx));
-        if (r < 0) {
-            q -= 1u;
-            r += (int32_t)nx;
-        } else if (r >= (int32_t)nx) {
-            q += 1u;
-            r -= (int32_t)nx;
-        }
-        const uint32_t sbx = (org & 0xFFFFu) + (uint32_t)r, sby = (org >> 16) + q;
+        uint32_t sbx, sby;
+        cand_xy(i, nx, sbx, sby);
+        sbx += org & 0xFFFFu;
+        sby += org >> 16;
         bool act = valid;
         if (any_check) {  // the reference's corner test for primitives spanning 3+ bin rows
             int32_t oc[3], odx[3], ody[3];
@@ -324,8 +385,7 @@ __device__ __forceinline__ void walk_bins(const FrameDev& F, uint32_t bins_x, ui
         const uint32_t slot = wave_add_slot_lds(ht, F.part_count, pkey, act);
         // the reservation, read here (pin keeps the read, and so its wait,
         // inside the pass instead of right after the atomic)
-        const uint32_t pbase = readlane_u32(pin(pres), 0);
-        const uint32_t ri = pbase + it;
+        const uint32_t ri = readlane_u32(pin(pres), 0) + it;
         if (valid && ri < cap) {
             const uint32_t p = first_p + ri, np = F.pair_total;
             F.pairs[p] = act ? orec : kNoPair;
@@ -334,10 +394,26 @@ __device__ __forceinline__ void walk_bins(const FrameDev& F, uint32_t bins_x, ui
                 F.pairs[2u * np + p] = slot;
             }
         }
-        if (base == 0 && lane == 0 && pbase + total > cap) {
-            atomicOr(&F.counters[C_FLAGS], FLAG_ENTRY_OVERFLOW);
-            atomicMax(&F.counters[clip ? C_CLIP_PAIR_NEED : C_PAIR_NEED], pbase + total);
+    }
+    const uint32_t pbase = readlane_u32(pin(pres), 0);
+    uint32_t at = pbase + total;
+    for (; bigs; bigs &= bigs - 1ull) {
+        const uint32_t src = (uint32_t)__builtin_ctzll(bigs);
+        int32_t oc[3], odx[3], ody[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            oc[k] = (int32_t)readlane_u32((uint32_t)c[k], src);
+            odx[k] = (int32_t)readlane_u32((uint32_t)dx[k], src);
+            ody[k] = (int32_t)readlane_u32((uint32_t)dy[k], src);
         }
+        const uint32_t n = readlane_u32(w.ncand, src);
+        walk_big(F, n, readlane_u32(pk_org, src), readlane_u32(pk_nx, src), readlane_u32(w.view_bins_x, src),
+                 readlane_u32(w.bin_base, src), readlane_u32(rec, src), oc, odx, ody, first_p, at, cap);
+        at += n;
+    }
+    if (lane == 0 && pbase + total_all > cap) {
+        atomicOr(&F.counters[C_FLAGS], FLAG_ENTRY_OVERFLOW);
+        atomicMax(&F.counters[clip ? C_CLIP_PAIR_NEED : C_PAIR_NEED], pbase + total_all);
     }
 }
 
@@ -542,6 +618,19 @@ __device__ __forceinline__ float lerp_kt(float a, float b, float t) { return a +
 // component-major with the lane innermost, so a wave's accesses to the same
 // component are conflict-free.
 constexpr uint32_t kClipThreads = 64;
+
+// Triangles a wave of k_clip takes at a time: 64 where that gives kClipWaves
+// waves, fewer below, so that a short queue is spread over more compute units
+// and each wave clips, sets up and bins less in a row; not below kClipMin,
+// because every wave reserves its records from one counter. Measured with 64
+// always / at least 4 / 8 / 16: 1280x720 cubes (251 triangles) 15.4 / 10.5 /
+// 10.6 / 10.8 us, 960x540 inside (4,887) 51.8 / 42.2 / 38.9 / 38.6; with
+// 10,460 triangles (1080p / 1 M) 14.9 at 64, 16.8 at 16, 14.4 at 27 (384 waves).
+constexpr uint32_t kClipMin = 16, kClipWaves = 384;
+__device__ __forceinline__ uint32_t clip_per_wave(uint32_t n)
+{
+    return min(max(n / kClipWaves, kClipMin), kClipThreads);
+}
 template <uint32_t NS>
 struct ClipPoly {
     static constexpr uint32_t kComps = 4 + NS;
@@ -612,11 +701,12 @@ __global__ __launch_bounds__(kClipThreads) void k_clip(FrameDev F)
     uint32_t* ht = s_hash + (threadIdx.x >> 6) * kWaveScratch;
     wave_hash_init(ht);
     const uint32_t n = F.counters[C_CLIPQ];
-    const uint32_t stride = gridDim.x * blockDim.x;
+    const uint32_t per = clip_per_wave(n);
+    const uint32_t stride = gridDim.x * per;
     const ClipPoly<NS> poly{ s_poly, threadIdx.x };
-    for (uint32_t base_i = blockIdx.x * blockDim.x; base_i < n; base_i += stride) {
+    for (uint32_t base_i = blockIdx.x * per; base_i < n; base_i += stride) {
         const uint32_t qi = base_i + threadIdx.x;
-        const bool active = qi < n;
+        const bool active = threadIdx.x < per && qi < n;
         uint32_t g = 0, d = 0, nfan = 0, pin_buf = 0;
         // what the fan triangles' set-up reads of the draw and its view,
         // loaded beside the vertices and handed on by shuffles

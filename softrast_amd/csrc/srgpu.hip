@@ -1145,7 +1145,7 @@ int run_frame(srg_ctx* ctx, bool noalloc)
         const uint32_t emit_blocks =
             std::max<uint32_t>(1, std::min<uint32_t>((F.pair_region_cap + emit_chunk - 1) / emit_chunk, 4096));
         const uint32_t clip_blocks = std::max<uint32_t>(
-            1, std::min<uint32_t>((NT + kClipThreads - 1) / kClipThreads, ctx->clip_resident[wide ? 2 : (narrow ? 0 : 1)]));
+            1, std::min<uint32_t>((NT + kClipMin - 1) / kClipMin, ctx->clip_resident[wide ? 2 : (narrow ? 0 : 1)]));
         const uint32_t init_blocks = std::min<uint32_t>(
             std::max<uint32_t>((kBinParts * TB + 255) / 256, (uint32_t)(off / 16 + 255) / 256), 1024);
         const uint32_t scan_blocks = (TB + kScanThreads - 1) / kScanThreads;
