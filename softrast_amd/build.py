@@ -69,10 +69,18 @@ def build_copy_calib():
     return out
 
 
+def build_rcp_check():
+    """Stand-alone device check of the RCPPS / RSQRTPS models (tests/test_gpu_rcp.py)."""
+    out = PKG / "rcp_check"
+    _run([HIPCC, *[f for f in HIP_FLAGS if f not in ("-shared", "-fPIC")], "-o", str(out), str(CSRC / "rcp_check.hip")])
+    return out
+
+
 def build_all():
     build_scene()
     build_gpu()
     build_copy_calib()
+    build_rcp_check()
 
 
 if __name__ == "__main__":

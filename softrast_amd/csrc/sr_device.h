@@ -16,13 +16,6 @@ constexpr uint32_t kMaxSlots = 4;         // attribute planes kept per primitive
 constexpr uint32_t kWideSlots = 8;        // ... by frames with a draw that reads eight varyings
 constexpr uint32_t kNoTex = 0xFFFFFFFFu;
 
-__device__ __constant__ uint32_t c_rcpps_table[2048] = {
-#include "rcpps_table.inc"
-};
-__device__ __constant__ uint32_t c_rsqrtps_table[4096] = {
-#include "rsqrtps_table.inc"
-};
-
 __device__ __forceinline__ uint32_t fbits(float f) { return __float_as_uint(f); }
 __device__ __forceinline__ float ffrom(uint32_t u) { return __uint_as_float(u); }
 
@@ -44,9 +37,36 @@ __device__ __forceinline__ int32_t cvtn_i32(float f)
 // _mm256_max_ps(a, b) = a > b ? a : b (second operand on NaN).
 __device__ __forceinline__ float maxps(float a, float b) { return a > b ? a : b; }
 
-// _mm256_rcp_ps as recorded on the reference's Intel host (Rasterizer.cpp:375-376):
-// table of the top 11 mantissa bits, exact exponent scaling, subnormal
-// results flushed to zero, zero/denormal -> inf, inf -> 0, NaN quieted.
+// _mm256_rcp_ps and _mm256_rsqrt_ps as recorded on the reference's Intel host
+// (Rasterizer.cpp:375-376, SponzaScene.cpp:67). Both recorded tables are a
+// function of the leading mantissa bits: RCPPS is 1 / m rounded to 2^-13, m
+// the middle of the input's cell of 2^-11 (the top 11 mantissa bits), RSQRTPS
+// 1 / sqrt(m) rounded to 2^-13, m the middle of the cell of the top 10
+// mantissa bits, the exponent scaled exactly. So they are computed with the
+// hardware's reciprocal and reciprocal square root instead of being looked
+// up: m set into the low bits, the instruction, a rounding constant, a mask.
+// Two of RCPPS's 2,048 values lie within 0.13 fp32 ulp of a rounding tie, on
+// either side of it; with m one ulp lower and the constant one lower than half
+// a unit every value comes out right. rcp_check.hip compares every cell at
+// every exponent with the recorded tables, on the device. The look-ups were
+// gathers from memory, 48 a pixel in the SponzaShader.
+
+// For inputs known to be positive normal numbers (rcpps: biased exponent <=
+// 251), with no special cases.
+__device__ __forceinline__ float rcpps_pos(float x)
+{
+    const float r = __builtin_amdgcn_rcpf(ffrom((fbits(x) & 0xFFFFF000u) | 0x7FFu));
+    return ffrom((fbits(r) + 0x3FFu) & 0xFFFFF800u);
+}
+__device__ __forceinline__ float rsqrtps_pos(float x)
+{
+    const float r = __builtin_amdgcn_rsqf(ffrom((fbits(x) & 0xFFFFE000u) | 0x1000u));
+    return ffrom((fbits(r) + 0x400u) & 0xFFFFF800u);
+}
+
+// Any input. RCPPS: subnormal results flushed to zero, zero / denormal -> inf,
+// inf -> 0, NaN quieted. RSQRTPS: +-0 and denormals -> +-inf, +inf -> +0, other
+// negatives -> the default NaN, NaN quieted.
 __device__ __forceinline__ float rcpps(float x)
 {
     const uint32_t u = fbits(x);
@@ -54,15 +74,10 @@ __device__ __forceinline__ float rcpps(float x)
     const uint32_t e = (u >> 23) & 255u;
     if (e == 255u) return ffrom((u & 0x7FFFFFu) ? (u | 0x00400000u) : sign);
     if (e == 0u) return ffrom(sign | 0x7F800000u);
-    const uint32_t t = c_rcpps_table[(u >> 12) & 2047u];
-    const int ne = (int)((t >> 23) & 255u) - ((int)e - 127);
+    const uint32_t t = fbits(rcpps_pos(ffrom((u & 0x7FFFFFu) | 0x3F800000u)));  // exponent field 126
+    const int ne = 253 - (int)e;
     return ffrom(ne <= 0 ? sign : (sign | ((uint32_t)ne << 23) | (t & 0x7FFFFFu)));
 }
-
-// _mm256_rsqrt_ps as recorded on the reference's Intel host (SponzaScene.cpp:67):
-// for x = 2^E * f, table T[E & 1][top 11 mantissa bits] scaled by
-// 2^-(E - (E & 1)) / 2 (always a normal result); +-0 and denormals -> +-inf,
-// +inf -> +0, other negatives -> the default NaN, NaN quieted.
 __device__ __forceinline__ float rsqrtps(float x)
 {
     const uint32_t u = fbits(x);
@@ -71,29 +86,7 @@ __device__ __forceinline__ float rsqrtps(float x)
     if (e == 0u) return ffrom((u & 0x80000000u) | 0x7F800000u);
     if (u & 0x80000000u) return ffrom(0xFFC00000u);
     if (e == 255u) return 0.0f;
-    const int ub = (int)e - 127, p = ub & 1;
-    const uint32_t t = c_rsqrtps_table[(uint32_t)p * 2048u + ((u >> 12) & 2047u)];
-    const int re = (int)((t >> 23) & 255u) - (ub - p) / 2;
-    return ffrom(((uint32_t)re << 23) | (t & 0x7FFFFFu));
-}
-
-// rsqrtps / rcpps for inputs known to be positive normal numbers (rcpps: biased
-// exponent <= 251), with no special cases: for those inputs they return the
-// same bits as the functions above (checked over every such input). The
-// table index of rsqrtps is the top 12 bits below the sign with the exponent's
-// low bit inverted (= T[E & 1]), the scale 2^-(E - (E & 1)) / 2 an integer
-// subtraction from the exponent field.
-__device__ __forceinline__ float rsqrtps_pos(float x)
-{
-    const uint32_t u = fbits(x);
-    const uint32_t t = c_rsqrtps_table[((u >> 12) & 0xFFFu) ^ 0x800u];
-    return ffrom(t - (((u + 0x00800000u) & 0xFF000000u) >> 1) + 0x20000000u);
-}
-__device__ __forceinline__ float rcpps_pos(float x)
-{
-    const uint32_t u = fbits(x);
-    const uint32_t t = c_rcpps_table[(u >> 12) & 2047u];
-    return ffrom(t - (u & 0x7F800000u) + 0x3F800000u);
+    return rsqrtps_pos(x);
 }
 
 // One channel of RGBA32SoA_To_RGBA8AoS (SIMDUtil.h:87-121): RNE(fma(c,255,.5)),
