@@ -27,12 +27,17 @@ __host__ __device__ constexpr uint32_t backend_threads(uint32_t S, uint32_t H) {
 // shades every kept fragment in submission order, so the final pixel is the
 // earliest-submitted fragment of largest depth. Key = depth bits << 32 |
 // (0xFFFFFFFE - order); an atomic max over the keys selects it. Initial key
-// from the depth already in the plane: D <= 0 -> 0, D NaN -> all ones
-// (nothing passes), D > 0 -> D's bits above every order field.
+// from the depth already in the plane: D <= 0 -> below every key of a depth
+// > 0 and above that of depth +0, D NaN -> above every key (nothing passes),
+// D > 0 -> D's bits above every order field; the low word of each names no
+// fragment. Initial keys are not negative as signed numbers, so a key of
+// negative depth (sign bit set) never wins a signed max: depths that cannot
+// be NaN need no test of their own.
+constexpr unsigned long long kKeyNone = 0xFFFFFFFFull;
 __device__ __forceinline__ unsigned long long init_key(float d0)
 {
-    if (d0 != d0) return ~0ull;
-    if (!(d0 > 0.0f)) return 0ull;
+    if (d0 != d0) return 0x7FFFFFFFFFFFFFFFull;
+    if (!(d0 > 0.0f)) return kKeyNone;
     return ((unsigned long long)fbits(d0) << 32) | 0xFFFFFFFFull;
 }
 
@@ -267,21 +272,16 @@ __device__ __forceinline__ uint32_t block_class(const uint32_t ct[3], const uint
     return rej <= 0 ? 0u : (full > 0 ? 2u : 1u);
 }
 
-// LDS slot of the key of strip-local pixel (x, y): rows of S keys, and inside
-// each group of G = min(S, 16) keys of a row the slot is rotated by
-// 2*(y>>3) + (x>>4) + 8*(y&1) (mod G). Keys are 8 bytes, so 16 consecutive
-// keys cover the LDS banks once.
-// Without the rotation the 64 lanes of a wave hit the same few banks: one
-// block per wave puts its 8 rows on the same banks, and one block per lane
-// puts the same pixel of every lane's block on the same bank. With it, a
-// block's 64 pixels fall on 16 bank pairs 4 apiece and the same pixel of the
-// 16 blocks of a 32x32 bin on 16 different bank pairs.
+// LDS slot of the key of strip-local pixel (x, y): rows of S keys, x's two low
+// bits exchanged by the block row. The lanes of a wave walk column pairs of
+// different block rows, all at the same row and column of their pair; rows are
+// a multiple of the banks long, so without the exchange the same column of
+// different block rows would meet on one bank. The second column's slot
+// differs from the first one's in bit 0 only, in every row.
 template <uint32_t S>
 __device__ __forceinline__ uint32_t key_slot(uint32_t x, uint32_t y)
 {
-    constexpr uint32_t G = S < 16u ? S : 16u;
-    const uint32_t rot = 2u * (y >> 3) + (x >> 4) + 8u * (y & 1u);
-    return y * S + (x & ~(G - 1u)) + ((x + rot) & (G - 1u));
+    return y * S + (x ^ ((y >> 3) & 3u));
 }
 
 // One primitive's tile-relative setup (Binning.cpp:423-451 re-basing) and its
@@ -370,36 +370,22 @@ __device__ __forceinline__ EntryRaster entry_raster(uint4 q0, uint4 q1, uint4 q2
 constexpr uint32_t kStageFields = 15;
 constexpr uint32_t kStageWords = (kStageFields + 1u) * 64u;
 
-template <uint32_t S, bool STATS>
-__device__ __forceinline__ void raster_wave(unsigned long long* keys, const EntryRaster& e, bool has, uint32_t sx0,
-                                            uint32_t sy0, unsigned long long& frags, uint32_t* stage)
+// One queue of raster_wave: the items of the lanes with n > 0. The entries are
+// staged; mark is the wave's 64-word mark array. FINITE: no entry's depth can
+// become NaN or infinite, so a signed max keeps out the depths <= 0 by itself;
+// otherwise every depth is tested. Without the test, and with two slot
+// addresses an item instead of four, a 1080p / 1 M frame issues 27.0 M VALU
+// instructions instead of 29.8 (69 -> 67 us; 64 views of 512x512 376 -> 365,
+// four 1440p views of 1 M 1,062 -> 991). Four columns an item with the edge
+// values of two columns in 16-bit halves and a second queue for the entries
+// that do not fit took more instructions (30.6 M, partial passes of two
+// queues) and 88 us.
+template <uint32_t S, bool FINITE, bool STATS>
+__device__ __forceinline__ void raster_items(unsigned long long* keys, const uint32_t* stage, uint32_t* mark, uint32_t n,
+                                             uint32_t first, uint32_t total, uint32_t sx0, uint32_t sy0,
+                                             unsigned long long& frags)
 {
     const uint32_t lane = lane_id();
-    const uint32_t cw = e.cx1 > e.cx0 ? e.cx1 - e.cx0 : 0u;
-    const uint32_t np = cw ? ((e.cx1 - 1u) >> 1) - (e.cx0 >> 1) + 1u : 0u;  // column pairs per block row
-    const uint32_t n = has ? e.nby * np : 0u;
-    const uint32_t incl = wave_incl_sum(n);
-    const uint32_t total = bcast(incl, 63);
-    // per-entry values the column workers need, packed; the first block row
-    // is cy0 rounded down to 8
-    // k / np == (k * magic) >> 16 for k < 512 when magic is ceil(2^16 / np)
-    // or one more (np <= 64); the 1-ulp reciprocal gives one of the two
-    const uint32_t npp = max(np, 1u);
-    const uint32_t magic = (uint32_t)(65536.0f * __builtin_amdgcn_rcpf((float)npp)) + 1u;
-    const uint32_t pk_cand = e.cx0 | (cw << 7) | (e.cy0 << 14) | (e.cy1 << 21) | ((e.tight ? 1u : 0u) << 28);
-    const uint32_t pk_div = magic | (npp << 17);
-    const uint32_t first = incl - n;
-    // each lane's entry into the wave's staging area: items read their
-    // owner's fields from there (a broadcast where lanes share an owner)
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // the previous entries' reads are issued
-    {
-        const uint32_t v[kStageFields] = { e.ct[0], e.ct[1], e.ct[2], e.dxu[0], e.dxu[1], e.dxu[2], e.dyu[0], e.dyu[1],
-                                           e.dyu[2], pk_cand, pk_div, fbits(e.zdx), fbits(e.zdy), fbits(e.zc0),
-                                           (uint32_t)e.low };
-#pragma unroll
-        for (uint32_t f = 0; f < kStageFields; ++f) stage[f * 64u + lane] = v[f];
-    }
-    uint32_t* mark = stage + kStageFields * 64u;
     uint32_t carry = 0;  // mark of the previous pass's last item
     for (uint32_t base = 0; base < total; base += 64) {
         const uint32_t it = base + lane;
@@ -436,20 +422,9 @@ __device__ __forceinline__ void raster_wave(unsigned long long* keys, const Entr
             thr = cls == 2u ? INT32_MIN : 0;
             walk_rows = cls != 0u;  // a rejected block draws nothing
         }
-        // key_slot of (x - sx0, yb + r - sy0): rows of S keys, the in-group
-        // rotation alternating with the row's parity (yb is a multiple of 8),
-        // so each column has one slot base for even rows and one for odd
-        // rows, and row r adds r * S keys (a constant offset). x is even, so
-        // x + 1 is in the same group of G keys.
-        constexpr uint32_t G = S < 16u ? S : 16u;
-        const uint32_t sxl = x - sx0, ybl = yb - sy0;
-        const uint32_t t = sxl + 2u * (ybl >> 3) + (sxl >> 4);
-        const uint32_t grp = ybl * S + (sxl & ~(G - 1u));
-        // byte offsets into keys of the four slot bases; grp is a multiple
-        // of G, so the odd rows' rotation by 8 flips bit 3 of the slot (G =
-        // 16) or changes nothing (G = 8)
-        const uint32_t b0e = pin(8u * (grp + (t & (G - 1u)))), b1e = pin(8u * (grp + ((t + 1u) & (G - 1u))));
-        const uint32_t b0o = pin(G == 16u ? b0e ^ 64u : b0e), b1o = pin(G == 16u ? b1e ^ 64u : b1e);
+        // byte offsets into keys of the pair's slots in its first row; row r
+        // adds r * S keys (a constant offset)
+        const uint32_t at0 = pin(8u * key_slot<S>(x - sx0, yb - sy0)), at1 = pin(at0 ^ 8u);
         char* const kb = reinterpret_cast<char*>(keys);
         // One walk down all eight rows of the block row. Rows and columns
         // outside cy0..cy1 x cx0..cx1 are walked too: for a primitive without
@@ -486,10 +461,15 @@ __device__ __forceinline__ void raster_wave(unsigned long long* keys, const Entr
                 if (!second) zmin = min(zmin, min((uint32_t)m0, (uint32_t)m1));
                 if (STATS) frags += (cov0 ? 1u : 0u) + (cov1 ? 1u : 0u);
                 const uint32_t ro = 8u * S * r;
-                auto* const k0 = reinterpret_cast<unsigned long long*>(kb + ((r & 1u) ? b0o : b0e) + ro);
-                auto* const k1 = reinterpret_cast<unsigned long long*>(kb + ((r & 1u) ? b1o : b1e) + ro);
-                if (cov0 & (ffrom((uint32_t)(q0 >> 32)) > 0.0f)) atomicMax(k0, q0);
-                if (cov1 & (ffrom((uint32_t)(q1 >> 32)) > 0.0f)) atomicMax(k1, q1);
+                auto put = [&](uint32_t at, unsigned long long key, bool cov) {
+                    if (FINITE) {
+                        if (cov) atomicMax(reinterpret_cast<long long*>(kb + at + ro), (long long)key);
+                    } else if (cov & (ffrom((uint32_t)(key >> 32)) > 0.0f)) {
+                        atomicMax(reinterpret_cast<unsigned long long*>(kb + at + ro), key);
+                    }
+                };
+                put(at0, q0, cov0);
+                put(at1, q1, cov1);
                 q0 = pin(((unsigned long long)fbits(ffrom((uint32_t)(q0 >> 32)) + zdy) << 32) | (uint32_t)q0);
                 q1 = pin(((unsigned long long)fbits(ffrom((uint32_t)(q1 >> 32)) + zdy) << 32) | (uint32_t)q1);
 #pragma unroll
@@ -506,6 +486,45 @@ __device__ __forceinline__ void raster_wave(unsigned long long* keys, const Entr
         // test decides it (rare; a wave-uniform branch)
         if (__ballot(zero))
             if (zero && block_class(ct, dxu, dyu, xb, yb) != 0u) (void)walk(std::true_type{});
+    }
+}
+
+template <uint32_t S, bool STATS>
+__device__ __forceinline__ void raster_wave(unsigned long long* keys, const EntryRaster& e, bool has, uint32_t sx0,
+                                            uint32_t sy0, unsigned long long& frags, uint32_t* stage)
+{
+    const uint32_t lane = lane_id();
+    const uint32_t cw = e.cx1 > e.cx0 ? e.cx1 - e.cx0 : 0u;
+    const uint32_t np = cw ? ((e.cx1 - 1u) >> 1) - (e.cx0 >> 1) + 1u : 0u;  // column pairs per block row
+    const uint32_t n = has ? e.nby * np : 0u;
+    // depths over a tile stay finite when the plane's terms are below 1e30
+    const bool finite = __builtin_fabsf(e.zc0) < 1.0e30f && __builtin_fabsf(e.zdx) < 1.0e30f && __builtin_fabsf(e.zdy) < 1.0e30f;
+    const uint32_t nf = finite ? n : 0u;
+    const uint32_t incl = wave_incl_sum(nf);
+    const uint32_t total = bcast(incl, 63);
+    // per-entry values the column workers need, packed; the first block row
+    // is cy0 rounded down to 8
+    // k / np == (k * magic) >> 16 for k < 512 when magic is ceil(2^16 / np)
+    // or one more (np <= 64); the 1-ulp reciprocal gives one of the two
+    const uint32_t npp = max(np, 1u);
+    const uint32_t magic = (uint32_t)(65536.0f * __builtin_amdgcn_rcpf((float)npp)) + 1u;
+    const uint32_t pk_cand = e.cx0 | (cw << 7) | (e.cy0 << 14) | (e.cy1 << 21) | ((e.tight ? 1u : 0u) << 28);
+    const uint32_t pk_div = magic | (npp << 17);
+    // each lane's entry into the wave's staging area: items read their
+    // owner's fields from there (a broadcast where lanes share an owner)
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // the previous entries' reads are issued
+    {
+        const uint32_t v[kStageFields] = { e.ct[0], e.ct[1], e.ct[2], e.dxu[0], e.dxu[1], e.dxu[2], e.dyu[0], e.dyu[1],
+                                           e.dyu[2], pk_cand, pk_div, fbits(e.zdx), fbits(e.zdy), fbits(e.zc0),
+                                           (uint32_t)e.low };
+#pragma unroll
+        for (uint32_t f = 0; f < kStageFields; ++f) stage[f * 64u + lane] = v[f];
+    }
+    uint32_t* mark = stage + kStageFields * 64u;
+    raster_items<S, true, STATS>(keys, stage, mark, nf, incl - nf, total, sx0, sy0, frags);
+    if (__ballot(n != nf)) {  // almost never
+        const uint32_t incl2 = wave_incl_sum(n - nf);
+        raster_items<S, false, STATS>(keys, stage, mark, n - nf, incl2 - (n - nf), bcast(incl2, 63), sx0, sy0, frags);
     }
 }
 
@@ -567,7 +586,7 @@ __global__ __launch_bounds__(backend_threads(S, H), backend_min_waves(S, H, STAT
 
         for (uint32_t p = tid; p < NPIX; p += T) {
             const uint32_t x = sx0 + p % S, y = sy0 + p / S;
-            keys[key_slot<S>(p % S, p / S)] = clear_d ? 0ull : init_key(global_ptr(V.depth)[tofs + y * kBin + x]);
+            keys[key_slot<S>(p % S, p / S)] = clear_d ? kKeyNone : init_key(global_ptr(V.depth)[tofs + y * kBin + x]);
         }
         __syncthreads();
 
@@ -598,7 +617,7 @@ __global__ __launch_bounds__(backend_threads(S, H), backend_min_waves(S, H, STAT
                 const uint32_t p = tid + (p0 + i) * T;
                 kk[i] = keys[key_slot<S>(p % S, p / S)];
                 const uint32_t lo = (uint32_t)kk[i];
-                win[i] = lo != 0xFFFFFFFFu && kk[i] != 0ull;
+                win[i] = lo != 0xFFFFFFFFu;
                 rec[i] = win[i] ? record_of_order(F, 0xFFFFFFFEu - lo) : 0u;
             }
 #pragma unroll

@@ -191,13 +191,23 @@ __device__ __forceinline__ void sample_wrap(const TexDev& T, float u, float v, f
     }
 }
 
-// UnlitDiffuseShader's sample (Viewer/Shaders.h:71-104), packed to RGBA8.
+// pack_channel of a value known to be in [0, 1.01] or NaN: the integer lies in
+// [0, 258], where the packs only saturate at 255; NaN gives 0 in both.
+__device__ __forceinline__ uint32_t pack_unit(float c)
+{
+    const float r = __builtin_rintf(__builtin_fmaf(c, 255.0f, 0.5f));
+    return min((uint32_t)__builtin_fmaxf(r, 0.0f), 255u);
+}
+
+// UnlitDiffuseShader's sample (Viewer/Shaders.h:71-104), packed to RGBA8. The
+// lerps of texel values in [0, 1] by fractions in [0, 1) stay there but for
+// rounding; a fraction is NaN when u or v is not finite.
 __device__ __forceinline__ uint32_t sample_unlit(const TexDev& T, float u, float v, float dudx, float dudy,
                                                  float dvdx, float dvdy)
 {
     float o[4];
     sample_wrap(T, u, v, dudx, dudy, dvdx, dvdy, o);
-    return pack_rgba(o[0], o[1], o[2], o[3]);
+    return pack_unit(o[0]) | (pack_unit(o[1]) << 8) | (pack_unit(o[2]) << 16) | (pack_unit(o[3]) << 24);
 }
 
 }  // namespace srg
