@@ -851,6 +851,16 @@ int run_frame(srg_ctx* ctx, bool noalloc)
         total_bins += (uint64_t)v.bins_x * v.bins_y;
     }
     if (total_bins * kBinParts >= 0xFFFFFFF0ull) return SRG_ERR_INVALID;  // (part, bin) indices are 32-bit
+    // A frame with so few bins that the GPU holds all their strips at once is
+    // split further where the configuration leaves it open: each workgroup
+    // then has less to do in a row. k_backend with 1 / 2 / 4 strips a bin:
+    // 320x180 (60 bins) 17.4 / 12.2 / 9.7 us, 960x540 (540) 54 / 39 / 38; past
+    // what is resident it loses: 1280x720 (960) 22 / 29 / 49, 1080p (2,040,
+    // 250 k triangles) 53 / 59 / 103. Recorded bin costs belong to one layout.
+    if (!ctx->cfg.wg_per_tile && L.bin_size == 32 && !autotune && ctx->cfg.tile_order != SRG_ORDER_LEARNED &&
+        !(ctx->cfg.flags & SRG_CFG_TILE_COSTS))
+        while (L.parts < 4 && total_bins * L.parts * 2 <= (uint64_t)ctx->num_cus * backend_min_waves(32, 32, false, false))
+            L.parts *= 2;
 
     // ---- draws, textures, front-end blocks ----
     std::vector<DrawDev> ddev(ctx->draws.size());
