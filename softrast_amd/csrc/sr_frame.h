@@ -119,7 +119,7 @@ struct FrameDev {
     uint32_t* bin_count;   // entries per bin (written by the scan)
     uint32_t* bin_start;   // total_bins + 1
     uint32_t* part_count;  // kBinParts x total_bins: entries per (part, bin); the count walks' slot cursors
-    uint32_t* part_off;    // kBinParts x total_bins: first entry of a part inside its bin's list
+    uint32_t* part_off;    // kBinParts x total_bins: first entry of a part of a bin's list
     uint32_t* entries;
     // (record, part-bin key, slot in the part's list) of every entry, as the
     // count walks find them: three arrays of pair_total words, one after
@@ -149,13 +149,16 @@ struct FrameDev {
 // every region holds a share of the frame's pairs.
 constexpr uint32_t kPairRegions = 256, kClipPairRegions = 8, kPairStride = 16;
 
-// A bin's counter and append cursor are split into kBinParts parts, the part
-// chosen by the entry's record (64 consecutive records share one), so the
-// atomics of a bin that many primitives land in spread over kBinParts
-// addresses. The scan sums the parts and lays them out one after another
-// inside the bin's entry list.
+// A bin's counter and entry list are split into kBinParts parts: two for each
+// of the chip's eight dies, the workgroup index giving the die (workgroups are
+// handed to the dies in turn) and the wave the half. So the atomics of a bin
+// that many primitives land in spread over kBinParts addresses, and a part's
+// entries, whose pairs k_scatter's workgroups of the same die take (a pair
+// region's index is its workgroups' modulo 8), are written through one die's
+// cache, where they fill lines. Only speed depends on which die runs what. The
+// scan lays the parts out one after another inside the bin's entry list.
 constexpr uint32_t kBinParts = 16;
-__host__ __device__ constexpr uint32_t part_of(uint32_t rec) { return (rec >> 6) & (kBinParts - 1u); }
+__device__ __forceinline__ uint32_t bin_part() { return (blockIdx.x & 7u) * 2u + ((threadIdx.x >> 6) & 1u); }
 
 __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 

@@ -268,11 +268,11 @@ __device__ __forceinline__ void cand_xy(uint32_t i, uint32_t nx, uint32_t& x, ui
 // stay as they are and k_setup<8> takes 32.7 or 39.2 us instead of 29.5 (1080p
 // / 250 k).
 constexpr uint32_t kBigCand = 64;
-__device__ __forceinline__ void walk_big(const FrameDev& F, uint32_t n, uint32_t org, uint32_t pn, uint32_t bins_x,
-                                         uint32_t bin_base, uint32_t rec, const int32_t c[3], const int32_t dx[3],
+__device__ __forceinline__ void walk_big(const FrameDev& F, uint32_t part, uint32_t n, uint32_t org, uint32_t pn,
+                                         uint32_t bins_x, uint32_t bin_base, uint32_t rec, const int32_t c[3], const int32_t dx[3],
                                          const int32_t dy[3], uint32_t first_p, uint32_t at, uint32_t cap)
 {
-    const uint32_t nx = pn & 0x7FFFFFFFu, part = part_of(rec) * F.total_bins;
+    const uint32_t nx = pn & 0x7FFFFFFFu;
     const bool check = (pn >> 31) != 0;
     for (uint32_t base = 0; base < n; base += 256) {
         uint32_t key[4], slot[4];
@@ -285,7 +285,7 @@ __device__ __forceinline__ void walk_big(const FrameDev& F, uint32_t n, uint32_t
             x += org & 0xFFFFu;
             y += org >> 16;
             act[k] = i < n && (!check || tile_accepts(c, dx, dy, (x >> F.bin_klog2) * kBin, (y >> F.bin_klog2) * kBin));
-            key[k] = part + bin_base + y * bins_x + x;
+            key[k] = part * F.total_bins + bin_base + y * bins_x + x;
             slot[k] = 0;
             if (act[k]) slot[k] = atomicAdd(&F.part_count[key[k]], 1u);
         }
@@ -350,6 +350,7 @@ __device__ __forceinline__ void walk_bins(const FrameDev& F, uint32_t bins_x, ui
     const uint32_t cap = clip ? F.clip_pair_cap : F.pair_region_cap;
     const uint32_t first_p = clip ? F.pair_regions * F.pair_region_cap + (region - F.pair_regions) * F.clip_pair_cap
                                   : region * F.pair_region_cap;
+    const uint32_t part = bin_part();
     uint32_t pres = 0;
     if (lane == 0 && total_all) pres = atomicAdd(&F.pair_count[region * kPairStride], total_all);
     uint32_t carry = 0;
@@ -381,7 +382,7 @@ __device__ __forceinline__ void walk_bins(const FrameDev& F, uint32_t bins_x, ui
                 act = false;
         }
         const uint32_t key = act ? bb + sby * vbx + sbx : 0u;
-        const uint32_t pkey = part_of(orec) * F.total_bins + key;  // the (part, bin) counter
+        const uint32_t pkey = part * F.total_bins + key;  // the (part, bin) counter
         const uint32_t slot = wave_add_slot_lds(ht, F.part_count, pkey, act);
         // the reservation, read here (pin keeps the read, and so its wait,
         // inside the pass instead of right after the atomic)
@@ -407,7 +408,7 @@ __device__ __forceinline__ void walk_bins(const FrameDev& F, uint32_t bins_x, ui
             ody[k] = (int32_t)readlane_u32((uint32_t)dy[k], src);
         }
         const uint32_t n = readlane_u32(w.ncand, src);
-        walk_big(F, n, readlane_u32(pk_org, src), readlane_u32(pk_nx, src), readlane_u32(w.view_bins_x, src),
+        walk_big(F, part, n, readlane_u32(pk_org, src), readlane_u32(pk_nx, src), readlane_u32(w.view_bins_x, src),
                  readlane_u32(w.bin_base, src), readlane_u32(rec, src), oc, odx, ody, first_p, at, cap);
         at += n;
     }
@@ -931,15 +932,16 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_apply(FrameDev F, const u
     const bool enq = q != 0;
     block_scan2(c, q, tc, tq);
     if (t < F.total_bins) {
-        F.bin_start[t] = blk[2 * blockIdx.x] + c;
+        const uint32_t start = blk[2 * blockIdx.x] + c;
+        F.bin_start[t] = start;
         if (enq) F.queue[blk[2 * blockIdx.x + 1] + q] = t;
-        uint32_t off = 0;  // the bin's parts, one after another
+        uint32_t off = start;  // the bin's parts, one after another
 #pragma unroll
         for (uint32_t k = 0; k < kBinParts; ++k) {
             F.part_off[k * F.total_bins + t] = off;
             off += F.part_count[k * F.total_bins + t];
         }
-        F.bin_count[t] = off;
+        F.bin_count[t] = off - start;
     }
 }
 
@@ -965,15 +967,16 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_single(FrameDev F)
         uint32_t sc = c, sq = enq ? 1u : 0u, tc, tq;
         block_scan2(sc, sq, tc, tq);
         if (t < nb) {
-            F.bin_start[t] = run_c + sc;
+            const uint32_t start = run_c + sc;
+            F.bin_start[t] = start;
             if (enq) F.queue[run_q + sq] = t;
-            uint32_t off = 0;  // the bin's parts, one after another
+            uint32_t off = start;  // the bin's parts, one after another
 #pragma unroll
             for (uint32_t k = 0; k < kBinParts; ++k) {
                 F.part_off[k * nb + t] = off;
                 off += cnt[k];
             }
-            F.bin_count[t] = off;
+            F.bin_count[t] = off - start;
         }
         run_c += tc;
         run_q += tq;
@@ -1061,8 +1064,8 @@ __global__ __launch_bounds__(kOrderBlock) void k_order_scatter(FrameDev F, const
     if (i < n) F.queue[atomicAdd(&off[bkt[i]], 1u)] = in_queue[i];
 }
 
-// Bin lists from the pairs of the count walks: entry (bin start + the part's
-// offset in the bin + the pair's slot) = record. An overflowed frame (pairs or
+// Bin lists from the pairs of the count walks: entry (the part's first entry
+// + the pair's slot) = record. An overflowed frame (pairs or
 // entries past the arena) is rendered again with larger arenas.
 //
 // grid: (regions, chunks); workgroup (r, c) takes chunks c, c + gridDim.y, ...
@@ -1091,8 +1094,7 @@ __global__ __launch_bounds__(256) void k_scatter(FrameDev F, uint32_t chunk)
             const uint32_t rec = F.pairs[p];
             if (rec == kNoPair) continue;  // a candidate bin the corner test rejected
             const uint32_t pkey = F.pairs[np + p], slot = F.pairs[2u * np + p];
-            const uint32_t key = pkey - part_of(rec) * F.total_bins;
-            F.entries[F.bin_start[key] + F.part_off[pkey] + slot] = rec;
+            F.entries[F.part_off[pkey] + slot] = rec;
         }
     }
 }
