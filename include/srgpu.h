@@ -239,16 +239,15 @@ int srg_end_frame_noalloc(srg_ctx* ctx);
 /* Copies the write plane's colour to linear RGBA8 rows (width*height*4 bytes),
  * swaps the planes, then calls on_finish(user) (Renderer.cpp:350-372).
  * Page-locked memory (hipHostMalloc) is written by the GPU itself, at the
- * host link's rate; pageable memory is written through page-locked chunks.
- * The same holds for srg_blit_async. */
+ * host link's rate; pageable memory is written through page-locked chunks. */
 int srg_blit(srg_ctx* ctx, srg_fb* fb, void* linear_rgba8, void (*on_finish)(void*), void* user);
 /* Blit (Renderer.cpp:350-372) with the reference's asynchrony: returns at
- * once; on a second stream the write plane is de-tiled into pinned memory
- * (overlapping the next frame), copied to linear_rgba8 (width*height*4
- * bytes) and on_finish(user) is called from a runtime thread, which must not
- * call into HIP. The planes are swapped at once. Like the reference, a blit
- * first waits for the previous blit, of the other plane, to finish; later
- * frames wait on the device until the blitted plane has been read.
+ * once; the write plane is de-tiled after the work submitted so far, the rows
+ * are copied to linear_rgba8 (width*height*4 bytes) on a second stream, beside
+ * the next frame, and on_finish(user) is called from a runtime thread, which
+ * must not call into HIP. The planes are swapped at once. Like the reference,
+ * a blit first waits for the previous blit, of the other plane, to finish;
+ * later frames write the blitted plane only after it has been read.
  * SRG_BLIT_BGRA exchanges red and blue on the way (the present swizzle of
  * Window_Win32::Flip, Viewer/Platform/Window_Win32.cpp:85-112). */
 #define SRG_BLIT_BGRA 1u

@@ -86,12 +86,13 @@ __global__ void k_fill_f32(float* p, float value, size_t n)
 // y0 .. y0 + rows - 1 to `linear`, row y0 first, a workgroup per row in turn.
 // With bgra, red and blue are exchanged on the way (the present swizzle of
 // Window_Win32::Flip, Viewer/Platform/Window_Win32.cpp:85-112).
-// `linear` is page-locked host memory and the kernel is bound by the host
-// link. V: pixels per lane and store, 4 where every row starts 16-byte
+// `linear` is page-locked host memory for a synchronous blit, and the kernel
+// is bound by the host link. V: pixels per lane and store, 4 where every row starts 16-byte
 // aligned (width a multiple of 4; a group of 4 never leaves its tile), so that
 // few waves keep the link full: 1920x1080 (8.3 MB) takes 162 us with 64
 // workgroups and V = 4, 170 with V = 1, 160 (the link's rate, 55 GB/s) with
-// 256 of either, all with the launch and the wait for it.
+// 256 of either, all with the launch and the wait for it. An asynchronous
+// blit's rows stay in device memory (6 us).
 template <uint32_t V>
 __global__ __launch_bounds__(256) void k_detile(const uint32_t* tiles, uint32_t* linear, uint32_t width, uint32_t y0,
                                                 uint32_t rows, uint32_t tiles_x, uint32_t bgra)
@@ -208,8 +209,8 @@ struct PlaneState {
     bool pending = false;
     int clear_colour = 0, clear_depth = 0;
     // asynchronous blit of this plane
-    uint32_t* pinned = nullptr;      // host rows written by the de-tile kernel
-    hipEvent_t read_done = nullptr;  // the plane's tiles have been read
+    uint32_t* rows = nullptr;        // the de-tiled rows, in device memory
+    uint32_t* pinned = nullptr;      // ... and on the host, for a target that is not page-locked
     hipEvent_t blit_done = nullptr;  // the callback has returned
     bool blit_pending = false;
     BlitJob job;
@@ -355,13 +356,6 @@ struct Carver {
     size_t left() const { return align_up(used, 256) >= cap ? 0 : cap - align_up(used, 256); }
 };
 
-// Work on the library stream that touches a plane waits until an
-// asynchronous blit of it has read its tiles.
-void stream_wait_blit_read(srg_ctx* ctx, PlaneState& p)
-{
-    if (p.blit_pending) (void)hipStreamWaitEvent(ctx->stream, p.read_done, 0);
-}
-
 // Host side: the blit of this plane, callback included, has finished.
 int finish_blit(PlaneState& p)
 {
@@ -376,10 +370,6 @@ void blit_host_fn(void* arg)
     if (j->src) std::memcpy(j->dst, j->src, j->bytes);
     if (j->cb) j->cb(j->user);
 }
-
-// Workgroups of an asynchronous blit: enough for the link, few enough to leave
-// the compute units to the frame that renders meanwhile.
-constexpr uint32_t kAsyncBlitBlocks = 64;
 
 // stop: an event that the kernel records (or null).
 void launch_detile(hipStream_t stream, uint32_t max_blocks, const uint32_t* tiles, uint32_t* out, const srg_fb* fb,
@@ -482,7 +472,6 @@ int copy_out(srg_ctx* ctx, void* dst, const uint32_t* src, size_t words)
 int flush_pending_clear(srg_ctx* ctx, srg_fb* fb, uint32_t plane)
 {
     PlaneState& ps = fb->planes[plane];
-    stream_wait_blit_read(ctx, ps);
     if (!ps.pending) return SRG_OK;
     const size_t n = (size_t)fb->tiles_x * fb->tiles_y * kTilePixels;
     const uint32_t b = ps.clear_value & 0xFFu;
@@ -1060,9 +1049,6 @@ int run_frame(srg_ctx* ctx, bool noalloc)
         want_clip = std::max<uint64_t>(want_clip, ctx->clip_cap);
         want_entries = std::max<uint64_t>(want_entries, ctx->entry_cap);
     }
-
-    // planes an asynchronous blit is still reading are written only after it
-    for (const ViewKey& v : views) stream_wait_blit_read(ctx, v.fb->planes[v.plane]);
 
     for (uint32_t attempt = 0;; ++attempt) {
         if (want_clip > 0xFFFFFFF0ull - NT || want_entries > 0xFFFFFFF0ull) return SRG_ERR_OVERFLOW;
@@ -1677,7 +1663,7 @@ void srg_fb_destroy(srg_ctx* ctx, srg_fb* fb)
         if (p.depth) (void)hipFree(p.depth);
         if (p.primid) (void)hipFree(p.primid);
         if (p.pinned) (void)hipHostFree(p.pinned);
-        if (p.read_done) (void)hipEventDestroy(p.read_done);
+        if (p.rows) (void)hipFree(p.rows);
         if (p.blit_done) (void)hipEventDestroy(p.blit_done);
     }
     ctx->fbs.erase(std::remove(ctx->fbs.begin(), ctx->fbs.end(), fb), ctx->fbs.end());
@@ -1716,7 +1702,6 @@ int srg_fb_write_tiles(srg_ctx* ctx, srg_fb* fb, uint32_t plane, const uint32_t*
     if (!fb_known(ctx, fb)) return SRG_ERR_HANDLE;
     const size_t n = (size_t)fb->tiles_x * fb->tiles_y * kTilePixels;
     PlaneState& p = fb->planes[plane];
-    stream_wait_blit_read(ctx, p);
     if (colour) {
         if (!p.colour) return SRG_ERR_INVALID;
         if (p.pending) p.clear_colour = 0;
@@ -1869,21 +1854,27 @@ int srg_blit_async(srg_ctx* ctx, srg_fb* fb, void* linear, uint32_t flags, void 
     if (!st) st = flush_pending_clear(ctx, fb, wp);
     if (st) return st;
     const size_t npx = (size_t)fb->width * fb->height;
-    uint32_t* dst = nullptr;
-    const bool direct = classify_dst(linear, npx * 4, &dst) == HostDst::pinned;
-    if (!direct) {
-        if (!p.pinned && hipHostMalloc((void**)&p.pinned, npx * 4, 0) != hipSuccess) return SRG_ERR_NOMEM;
-        HIP_TRY(hipHostGetDevicePointer((void**)&dst, p.pinned, 0));
+    uint32_t* dev = nullptr;
+    const bool direct = classify_dst(linear, npx * 4, &dev) == HostDst::pinned;
+    if (!direct && !p.pinned && hipHostMalloc((void**)&p.pinned, npx * 4, 0) != hipSuccess) {
+        p.pinned = nullptr;
+        return SRG_ERR_NOMEM;
     }
-    if (!p.read_done) HIP_TRY(hipEventCreateWithFlags(&p.read_done, hipEventDisableTiming));
+    if (!p.rows && hipMalloc((void**)&p.rows, npx * 4) != hipSuccess) {
+        p.rows = nullptr;
+        return SRG_ERR_NOMEM;
+    }
     if (!p.blit_done) HIP_TRY(hipEventCreateWithFlags(&p.blit_done, hipEventDisableTiming));
-    // the copy stream starts once the frame that wrote the plane is done
+    // The rows are de-tiled on the library stream (6 us at 1080p), so later
+    // frames are ordered after it, and copied out by the second stream's copy
+    // engine. A kernel that writes the rows over the host link itself holds up
+    // every kernel of the next frame: a small kernel launched beside it was
+    // done after 151 us, as the 8.3 MB were, instead of 10 beside the copy.
+    launch_detile(ctx->stream, 256, p.colour, p.rows, fb, 0, fb->height, (flags & SRG_BLIT_BGRA) != 0, nullptr);
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(ctx->ev[3], ctx->stream));
     HIP_TRY(hipStreamWaitEvent(ctx->copy_stream, ctx->ev[3], 0));
-    launch_detile(ctx->copy_stream, kAsyncBlitBlocks, p.colour, dst, fb, 0, fb->height, (flags & SRG_BLIT_BGRA) != 0,
-                  nullptr);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipEventRecord(p.read_done, ctx->copy_stream));
+    HIP_TRY(hipMemcpyAsync(direct ? linear : p.pinned, p.rows, npx * 4, hipMemcpyDeviceToHost, ctx->copy_stream));
     p.job = BlitJob{ linear, direct ? nullptr : p.pinned, npx * 4, on_finish, user };
     HIP_TRY(hipLaunchHostFunc(ctx->copy_stream, blit_host_fn, &p.job));
     HIP_TRY(hipEventRecord(p.blit_done, ctx->copy_stream));
