@@ -50,7 +50,7 @@ struct ViewDev {
 };
 
 enum : uint32_t {
-    C_CLIPQ = 0,       // clipped triangles queued for the slow path
+    C_CLIPQ = 0,       // clipped triangles queued for the slow path (k_clip's sum of its lists)
     C_CLIPREC = 1,     // records allocated by the slow path
     C_FLAGS = 2,       // error / overflow bits
     C_QLEN = 3,        // back-end queue length
@@ -113,7 +113,7 @@ struct FrameDev {
     const SponzaDev* sponza;  // SponzaShader constants (wide frames only)
     const uint32_t* sched_gate;  // learned order: [1] != 0 on frames that predict and record (else null)
     uint32_t* rec_meta;    // draw index (written only for slots that hold a primitive)
-    uint2* clip_queue;     // per triangle routed to the clipper: (global triangle id, draw index)
+    uint2* clip_queue;     // per triangle routed to the clipper: (global triangle id, draw index), kClipLists lists
     uint32_t* clip_base;   // per global triangle: first fan record (relative to ntris)
     uint32_t* clip_order;  // per fan record: order key
     uint32_t* bin_count;   // entries per bin (written by the scan)
@@ -148,6 +148,32 @@ struct FrameDev {
 // as many regions as k_setup has workgroups, at most kPairRegions, so that
 // every region holds a share of the frame's pairs.
 constexpr uint32_t kPairRegions = 256, kClipPairRegions = 8, kPairStride = 16;
+
+// The clipper's queue is kClipLists lists, each with a counter on a line of
+// its own (the second word of a pair region's), because atomics on one address
+// take about 6.5 ns each: with one counter, 2560x1440 / 4 M triangles, most of
+// whose 62,500 waves hold a clipped triangle, spent its time there. k_setup
+// with one / 16 / 32 / 64 lists: 401 / 312 / 313 / 312 us there, 207 / 179 /
+// 180 / 180 for 64 views, 88 / 76 / 77 / 76 for 24 mixed views, 20.6 / 12.6 /
+// 12.5 / 12.6 at 960x540 inside the geometry; k_clip, which reads every
+// counter first, pays 0.3 - 0.7 us with 16, 1.0 with 64. Triangle g belongs to
+// list (g / 256) mod kClipLists; a list has room for all of its triangles, so
+// none overflows, and together they take one slot per triangle.
+constexpr uint32_t kClipLists = 16, kClipChunkLog2 = 8;
+__device__ __forceinline__ uint32_t clip_list(uint32_t g) { return (g >> kClipChunkLog2) % kClipLists; }
+__device__ __forceinline__ uint32_t* clip_count(const FrameDev& F, uint32_t list)
+{
+    return F.pair_count + list * (kPairRegions / kClipLists) * kPairStride + 1u;
+}
+// First queue slot of a list: the triangles of the lists before it, each
+// holding every kClipLists-th chunk of 256 triangles, the last chunk cut short.
+__device__ __forceinline__ uint32_t clip_list_base(uint32_t ntris, uint32_t list)
+{
+    const uint32_t chunks = (ntris + (1u << kClipChunkLog2) - 1u) >> kClipChunkLog2;
+    const uint32_t before = list * (chunks / kClipLists) + min(list, chunks % kClipLists);
+    const uint32_t cut = list > (chunks - 1u) % kClipLists ? (chunks << kClipChunkLog2) - ntris : 0u;
+    return (before << kClipChunkLog2) - cut;
+}
 
 // A bin's counter and entry list are split into kBinParts parts: two for each
 // of the chip's eight dies, the workgroup index giving the die (workgroups are

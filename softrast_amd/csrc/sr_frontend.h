@@ -596,19 +596,29 @@ __global__ __launch_bounds__(kSetupThreads) void k_setup(FrameDev F, const Setup
         }
         // a slot without a primitive is never referenced: nothing is written there
         if (survive) write_record<NS>(F, g, s, d);
-        // The clip queue's slots (at most one per triangle: never overflows),
-        // reserved here and filled after the bins are walked, so that the
-        // reservation's round trip overlaps the walk.
+        // The clip queue's slots, reserved here and filled after the bins are
+        // walked, so that the reservation's round trip overlaps the walk. The
+        // wave's triangles lie in one list or in two: the first lane's, whose
+        // slots that lane reserves, and the last lane's.
         const unsigned long long cm = __ballot(clipped);
+        const bool second = clip_list(g) != clip_list(readlane_u32(g, 0));
+        const unsigned long long cm2 = __ballot(clipped && second);
         uint32_t q = 0;
-        if (cm && lane_id() == 0) q = atomicAdd(&F.counters[C_CLIPQ], (uint32_t)__popcll(cm));
+        if (cm) {
+            const uint32_t want = (uint32_t)__popcll(lane_id() ? cm2 : cm ^ cm2);
+            if (want && (lane_id() == 0 || lane_id() == 63)) q = atomicAdd(clip_count(F, clip_list(g)), want);
+        }
 
         if (stats) block_stats_add(&bs, set_up ? reference_tile_entries(s) : 0u, set_up ? 1u : 0u);
         walk_bins(F, V.bins_x, V.bin_base, survive, s.c, s.dx, s.dy, s.xmin, s.xmax, s.ymin, s.ymax, g, ht, false);
-        if (clipped)
-            F.clip_queue[readlane_u32(pin(q), 0) + __builtin_amdgcn_mbcnt_hi((uint32_t)(cm >> 32),
-                                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)cm, 0))] =
+        q = pin(q);  // by every lane: the two that hold the reservations need not be clipped
+        const uint32_t q_first = readlane_u32(q, 0), q_second = readlane_u32(q, 63);
+        if (clipped) {
+            const unsigned long long peers = second ? cm2 : cm ^ cm2;
+            F.clip_queue[clip_list_base(F.ntris, clip_list(g)) + (second ? q_second : q_first) +
+                         __builtin_amdgcn_mbcnt_hi((uint32_t)(peers >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)peers, 0))] =
                 make_uint2(g, d);
+        }
     }
     if (stats) {
         __syncthreads();
@@ -714,19 +724,32 @@ __global__ __launch_bounds__(kClipThreads) void k_clip(FrameDev F)
     __shared__ uint32_t s_hash[kClipThreads / 64 * kWaveScratch];
     uint32_t* ht = s_hash + (threadIdx.x >> 6) * kWaveScratch;
     wave_hash_init(ht);
-    const uint32_t n = F.counters[C_CLIPQ];
+    // the lists' lengths, one a lane, and how far they reach in the whole queue
+    const uint32_t list_n = lane_id() < kClipLists ? *clip_count(F, lane_id()) : 0u;
+    const uint32_t list_end = wave_incl_sum(list_n), list_first = list_end - list_n;
+    const uint32_t n = readlane_u32(list_end, 63);
+    if (blockIdx.x == 0 && threadIdx.x == 0) F.counters[C_CLIPQ] = n;
     const uint32_t per = clip_per_wave(n);
     const uint32_t stride = gridDim.x * per;
     const ClipPoly<NS> poly{ s_poly, threadIdx.x };
     for (uint32_t base_i = blockIdx.x * per; base_i < n; base_i += stride) {
         const uint32_t qi = base_i + threadIdx.x;
         const bool active = threadIdx.x < per && qi < n;
+        // the list that holds entry qi, and the entry's slot
+        uint32_t list = 0, list_hi = kClipLists - 1u;
+#pragma unroll
+        for (uint32_t span = kClipLists; span > 1u; span >>= 1) {
+            const uint32_t mid = (list + list_hi) >> 1;
+            if (__shfl(list_end, (int)mid, 64) > qi) list_hi = mid;
+            else list = min(mid + 1u, kClipLists - 1u);
+        }
+        const uint32_t slot = clip_list_base(F.ntris, list) + qi - __shfl(list_first, (int)list, 64);
         uint32_t g = 0, d = 0, nfan = 0, pin_buf = 0;
         // what the fan triangles' set-up reads of the draw and its view,
         // loaded beside the vertices and handed on by shuffles
         uint32_t wh = 0, nslots = 0, bins_x = 0, bin_base = 0;
         if (active) {
-            const uint2 e = F.clip_queue[qi];
+            const uint2 e = F.clip_queue[slot];
             g = e.x;
             d = e.y;
             const DrawDev& D = F.draws[d];
