@@ -9,10 +9,10 @@
 // primitive record so the loads overlap; the entries' column pairs of 8x8
 // block rows then form a queue the wave takes 64 at a time, a lane per pair
 // walking its eight rows (RasterizeTrisInBin_OutputFragments and
-// ComputeBlockMask8x8, Rasterizer.cpp:97-304). Then each lane resolves its pixels (the key names
-// the fragment the reference would have shaded last) and shades them
-// (ComputeInterpolantsDrawCallImpl :306-419, Shaders.h, Texture.cpp),
-// writing RGBA8 and depth once.
+// ComputeBlockMask8x8, Rasterizer.cpp:97-304). Then each lane resolves its
+// pixels (the key names the fragment the reference would have shaded last) and
+// shades them (ComputeInterpolantsDrawCallImpl :306-419, Shaders.h,
+// Texture.cpp), writing RGBA8 and depth once.
 #pragma once
 #include <type_traits>
 

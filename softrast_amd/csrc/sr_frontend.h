@@ -3,7 +3,8 @@
 //   k_setup  one lane per triangle of a setup group (draws sharing their
 //            geometry), fetched once and set up for each draw of the group;
 //            unclipped survivors are written to their own record slot,
-//            clipped triangles are queued for k_clip; bin entries are counted
+//            clipped triangles are queued for k_clip (in kClipLists lists);
+//            bin entries are counted
 //   k_clip   slow path over the queued triangles: Sutherland-Hodgman clip,
 //            fan, setup of each fan triangle, bin counts
 //   k_scan   exclusive scan of bin counts + the back end's work queue

@@ -1,11 +1,14 @@
 // srgpu.hip -- MI355X (gfx950) sort-middle rasteriser behind the C ABI of
 // include/srgpu.h.
 //
-// A frame is six launches on one stream:
-//   k_frame_init  zero counters and per-bin arrays (a fill kernel, no memset)
+// A frame is six launches on one stream (a few more with many bins or a sorted
+// queue):
+//   k_frame_init  zero counters and per-bin arrays (a fill kernel, no memset),
+//                 fetch the frame's tables from page-locked host memory
 //   k_setup       one lane per submitted triangle (sr_frontend.h)
 //   k_clip        slow path for triangles crossing a clip plane
-//   k_scan_*      bin offsets and the back end's work queue (three passes)
+//   k_scan_*      bin offsets and the back end's work queue (three passes, or
+//                 one for at most 4,096 bins); the frame's counters to the host
 //   k_scatter     bin lists from the (record, bin) pairs the count walks found
 //   k_backend<S>  persistent raster + resolve + shade per S x S bin (sr_backend.h)
 //
@@ -40,9 +43,10 @@ namespace srg {
 // (graph-safe). With the learned order, gate[1] says whether this frame
 // predicts and records (every `every`-th frame, counted in gate[0] on the
 // device so that replayed graphs count too).
-// Counter words of a frame: the C_NCOUNTERS frame counters (copied back to
-// the host), then from word 64 the counters of the pair regions (at most
-// kPairRegions for k_setup, kClipPairRegions more for k_clip).
+// Counter words of a frame: the C_NCOUNTERS frame counters (written to the host
+// by the scan), then from word 64 the counters of the pair regions (at most
+// kPairRegions for k_setup, kClipPairRegions more for k_clip), the second word
+// of every sixteenth counting a list of the clipper's queue.
 constexpr uint32_t kPairCounterBase = 64,
                    kCounterWords = kPairCounterBase + (kPairRegions + kClipPairRegions) * kPairStride;
 

@@ -1,8 +1,8 @@
 """Turn the recorded RCPPS fixture (rcpps_table.txt) into C initialiser lists.
 
 Writes oracle/rcpps_table.inc (used by the CPU oracle) and
-softrast_amd/csrc/rcpps_table.inc (compiled into the HIP library). Both hold
-the same 2048 words: bits of rcp(1 + i/2048) as observed on an Intel host
+softrast_amd/csrc/rcpps_table.inc (what rcp_check.hip holds the library's
+formula against, word for word). Both hold the same 2048 words: bits of rcp(1 + i/2048) as observed on an Intel host
 (see gen_rcpps_table.c). tests/test_oracle_kat.py checks both against the fixture.
 """
 import pathlib
