@@ -51,25 +51,21 @@ __device__ __forceinline__ uint32_t record_of_order(const FrameDev& F, uint32_t 
 // one pixel: all eight varyings (0-2 position, 3-5 normal, 6-7 uv), the uv
 // derivatives from the slots at uv_offset, sun, 16 point lights by
 // RSQRTPS / RCPPS, ambient, times the texture sample.
-__device__ __forceinline__ uint32_t shade_sponza(const FrameDev& F, const DrawDev& D, uint32_t rec, int32_t X0,
+__device__ __forceinline__ uint32_t shade_sponza(const FrameDev& F, const DrawDev& D, uint32_t rec, uint4 q3, int32_t X0,
                                                  int32_t Y0, uint32_t px, uint32_t py)
 {
     if (D.tex == kNoTex) return 0xFFFFFFFFu;
     const TexDev& T = F.texs[D.tex];
     if (T.empty) return 0xFFFFFFFFu;
-    const float* Sp = F.rec_shade + (size_t)rec * F.shade_stride;
+    const float4* Sp = F.rec_shade + (size_t)rec * F.shade_quads;
     const float4* Ep = F.rec_ext + (size_t)rec * 3;
-    const float4 s0 = make_float4(Sp[0], Sp[1], Sp[2], Sp[3]), s1 = make_float4(Sp[4], Sp[5], Sp[6], Sp[7]);
-    const float4 s2 = make_float4(Sp[8], Sp[9], Sp[10], Sp[11]), s3 = make_float4(Sp[12], Sp[13], Sp[14], 0.0f);
-    const float4 e0 = Ep[0], e1 = Ep[1], e2 = Ep[2];
-    const uint4 q2 = F.rec_raster[(size_t)rec * 4 + 2];
-    const uint4 q3 = F.rec_raster[(size_t)rec * 4 + 3];
-    const float sx = (float)X0 - ffrom(q2.w), sy = (float)Y0 - ffrom(q3.x);
+    const float4 s0 = Sp[0], s1 = Sp[1], s2 = Sp[2], s3 = Sp[3], e0 = Ep[0], e1 = Ep[1], e2 = Ep[2];
+    const float sx = (float)X0 - ffrom(q3.x), sy = (float)Y0 - ffrom(q3.y);
     const float wdx = s0.x, wdy = s0.y;
-    const float wc = wdx * sx + wdy * sy + s0.z;
-    const float pdx[kWideSlots] = { s0.w, s1.z, s2.y, s3.x, e0.x, e0.w, e1.z, e2.y };
-    const float pdy[kWideSlots] = { s1.x, s1.w, s2.z, s3.y, e0.y, e1.x, e1.w, e2.z };
-    const float pf0[kWideSlots] = { s1.y, s2.x, s2.w, s3.z, e0.z, e1.y, e2.x, e2.w };
+    const float wc = wdx * sx + wdy * sy + ffrom(q3.w);
+    const float pdx[kWideSlots] = { s0.z, s1.y, s2.x, s2.w, e0.x, e0.w, e1.z, e2.y };
+    const float pdy[kWideSlots] = { s0.w, s1.z, s2.y, s3.x, e0.y, e1.x, e1.w, e2.z };
+    const float pf0[kWideSlots] = { s1.x, s1.w, s2.z, s3.y, e0.z, e1.y, e2.x, e2.w };
     const float X = (float)px, Y = (float)py;
     const float iq = 1.0f / __builtin_fmaf(X, wdx, __builtin_fmaf(Y, wdy, wc));
     float pc[kWideSlots], var[kWideSlots];
@@ -157,32 +153,30 @@ template <bool WIDE>
 __device__ __forceinline__ uint32_t shade_pixel(const FrameDev& F, uint32_t rec, int32_t X0, int32_t Y0, uint32_t px,
                                                 uint32_t py)
 {
-    const uint32_t d = F.rec_meta[rec];
-    const DrawDev& D = F.draws[d];
-    if (WIDE && D.shader == SRG_SHADER_SPONZA) return shade_sponza(F, D, rec, X0, Y0, px, py);
-    // shade record: (wdx, wdy, w0), then (dx, dy, value) of each kept slot
-    const float* Sp = F.rec_shade + (size_t)rec * F.shade_stride;
-    const float4 s0 = make_float4(Sp[0], Sp[1], Sp[2], Sp[3]), s1 = make_float4(Sp[4], Sp[5], Sp[6], Sp[7]);
-    const float pf01 = Sp[8];
-    const uint32_t* Rw = (const uint32_t*)(F.rec_raster + (size_t)rec * 4);
+    const uint4 q3 = F.rec_raster[(size_t)rec * 4 + 3];  // r0, draw, 1/w at v0
+    const DrawDev& D = F.draws[q3.z];
+    if (WIDE && D.shader == SRG_SHADER_SPONZA) return shade_sponza(F, D, rec, q3, X0, Y0, px, py);
+    // shade record: 1/w's steps, then (dx, dy, value) of each kept slot
+    const float4* Sp = F.rec_shade + (size_t)rec * F.shade_quads;
+    const float4 s0 = Sp[0], s1 = Sp[1];
     // plane constants re-based to the tile origin (Binning.cpp:435-452)
-    const float sx = (float)X0 - ffrom(Rw[11]), sy = (float)Y0 - ffrom(Rw[12]);
+    const float sx = (float)X0 - ffrom(q3.x), sy = (float)Y0 - ffrom(q3.y);
     const float wdx = s0.x, wdy = s0.y;
-    const float wc = wdx * sx + wdy * sy + s0.z;
+    const float wc = wdx * sx + wdy * sy + ffrom(q3.w);
     const float X = (float)px, Y = (float)py;
     const float iq = 1.0f / __builtin_fmaf(X, wdx, __builtin_fmaf(Y, wdy, wc));
     // slots 0 and 1: the sampled (u, v), the normal's x, y, or the shown uv
-    float tdx[2] = { s0.w, s1.z }, tdy[2] = { s1.x, s1.w }, tc[2], tv[2];
-    tc[0] = tdx[0] * sx + tdy[0] * sy + s1.y;
-    tc[1] = tdx[1] * sx + tdy[1] * sy + pf01;
+    float tdx[2] = { s0.z, s1.y }, tdy[2] = { s0.w, s1.z }, tc[2], tv[2];
+    tc[0] = tdx[0] * sx + tdy[0] * sy + s1.x;
+    tc[1] = tdx[1] * sx + tdy[1] * sy + s1.w;
     tv[0] = iq * __builtin_fmaf(tdy[0], Y, __builtin_fmaf(tdx[0], X, tc[0]));
     tv[1] = iq * __builtin_fmaf(tdy[1], Y, __builtin_fmaf(tdx[1], X, tc[1]));
     const float u = tv[0], v = tv[1];
     switch (D.shader) {
     case SRG_SHADER_VISUALIZE_NORMALS: {
-        const float4 s2 = make_float4(Sp[8], Sp[9], Sp[10], Sp[11]);
-        const float c2 = s2.y * sx + s2.z * sy + s2.w;
-        const float n2 = iq * __builtin_fmaf(s2.z, Y, __builtin_fmaf(s2.y, X, c2));
+        const float4 s2 = Sp[2];
+        const float c2 = s2.x * sx + s2.y * sy + s2.z;
+        const float n2 = iq * __builtin_fmaf(s2.y, Y, __builtin_fmaf(s2.x, X, c2));
         return pack_rgba(__builtin_fmaf(u, 0.5f, 0.5f), __builtin_fmaf(v, 0.5f, 0.5f), __builtin_fmaf(n2, 0.5f, 0.5f),
                          1.0f);
     }
@@ -194,10 +188,10 @@ __device__ __forceinline__ uint32_t shade_pixel(const FrameDev& F, uint32_t rec,
     const TexDev& T = F.texs[D.tex];
     if (T.empty) return 0xFFFFFFFFu;
     if (D.deriv_slot != 0) {  // uv_offset != 6: derivatives from slots 2 and 3
-        const float4 s2 = make_float4(Sp[8], Sp[9], Sp[10], Sp[11]), s3 = make_float4(Sp[12], Sp[13], Sp[14], 0.0f);
-        tdx[0] = s2.y; tdy[0] = s2.z; tdx[1] = s3.x; tdy[1] = s3.y;
-        tc[0] = tdx[0] * sx + tdy[0] * sy + s2.w;
-        tc[1] = tdx[1] * sx + tdy[1] * sy + s3.z;
+        const float4 s2 = Sp[2], s3 = Sp[3];
+        tdx[0] = s2.x; tdy[0] = s2.y; tdx[1] = s2.w; tdy[1] = s3.x;
+        tc[0] = tdx[0] * sx + tdy[0] * sy + s2.z;
+        tc[1] = tdx[1] * sx + tdy[1] * sy + s3.y;
         tv[0] = iq * __builtin_fmaf(tdy[0], Y, __builtin_fmaf(tdx[0], X, tc[0]));
         tv[1] = iq * __builtin_fmaf(tdy[1], Y, __builtin_fmaf(tdx[1], X, tc[1]));
     }
@@ -303,12 +297,12 @@ __device__ __forceinline__ EntryRaster entry_raster(uint4 q0, uint4 q1, uint4 q2
                                                     int32_t Y0, uint32_t sx0, uint32_t sy0, uint32_t S, uint32_t H)
 {
     EntryRaster e;
-    e.dxu[0] = q0.w; e.dxu[1] = q1.x; e.dxu[2] = q1.y;
-    e.dyu[0] = q1.z; e.dyu[1] = q1.w; e.dyu[2] = q2.x;
+    e.dxu[0] = q0.w; e.dxu[1] = q1.x; e.dxu[2] = 0u - (q0.w + q1.x);
+    e.dyu[0] = q1.y; e.dyu[1] = q1.z; e.dyu[2] = 0u - (q1.y + q1.z);
     const uint32_t c[3] = { q0.x, q0.y, q0.z };
 #pragma unroll
     for (int k = 0; k < 3; ++k) e.ct[k] = c[k] + (e.dxu[k] * (uint32_t)Y0 + e.dyu[k] * (uint32_t)X0);
-    const int32_t xmin = q2.y & 0x3FFF, xmax = (q2.y >> 16) & 0x3FFF, ymin = q2.z & 0x3FFF, ymax = (q2.z >> 16) & 0x3FFF;
+    const int32_t xmin = q1.w & 0x3FFF, xmax = (q1.w >> 16) & 0x3FFF, ymin = q2.x & 0x3FFF, ymax = (q2.x >> 16) & 0x3FFF;
     const uint32_t bminx = (uint32_t)clampi(xmin - X0, 0, 64), bmaxx = (uint32_t)clampi(xmax - X0, 0, 64);
     const uint32_t bminy = (uint32_t)clampi(ymin - Y0, 0, 64), bmaxy = (uint32_t)clampi(ymax - Y0, 0, 64);
     e.xs = max(bminx & ~7u, sx0);
@@ -316,13 +310,13 @@ __device__ __forceinline__ EntryRaster entry_raster(uint4 q0, uint4 q1, uint4 q2
     e.ys = max(bminy & ~7u, sy0);
     e.ye = min(bmaxy, sy0 + H);
     // walked pixels: whole blocks from xs while xb < xe (xs, ys are multiples of 8)
-    e.tight = ((q2.y >> 14) & 1u) != 0;
+    e.tight = ((q1.w >> 14) & 1u) != 0;
     const int32_t wx1 = e.xe > e.xs ? (int32_t)(e.xs + ((e.xe - e.xs + 7u) & ~7u)) : (int32_t)e.xs;
     const int32_t wy1 = e.ye > e.ys ? (int32_t)(e.ys + ((e.ye - e.ys + 7u) & ~7u)) : (int32_t)e.ys;
     if (e.tight) {
-        e.cx0 = (uint32_t)max((int32_t)e.xs, xmin - (int32_t)((q2.y >> 15) & 1u) - X0);
-        e.cy0 = (uint32_t)max((int32_t)e.ys, ymin - (int32_t)((q2.z >> 14) & 1u) - Y0);
-        const int32_t bx1 = ((q2.y >> 30) & 1u) ? wx1 : xmax - X0 + 1, by1 = ((q2.z >> 30) & 1u) ? wy1 : ymax - Y0 + 1;
+        e.cx0 = (uint32_t)max((int32_t)e.xs, xmin - (int32_t)((q1.w >> 15) & 1u) - X0);
+        e.cy0 = (uint32_t)max((int32_t)e.ys, ymin - (int32_t)((q2.x >> 14) & 1u) - Y0);
+        const int32_t bx1 = ((q1.w >> 30) & 1u) ? wx1 : xmax - X0 + 1, by1 = ((q2.x >> 30) & 1u) ? wy1 : ymax - Y0 + 1;
         e.cx1 = (uint32_t)max((int32_t)e.cx0, min(wx1, bx1));
         e.cy1 = (uint32_t)max((int32_t)e.cy0, min(wy1, by1));
     } else {
@@ -335,11 +329,11 @@ __device__ __forceinline__ EntryRaster entry_raster(uint4 q0, uint4 q1, uint4 q2
     e.by0 = e.cy0 & ~7u;
     e.nbx = e.cx1 > e.cx0 ? ((e.cx1 - 1u) >> 3) - (e.cx0 >> 3) + 1u : 0u;
     e.nby = e.cy1 > e.cy0 ? ((e.cy1 - 1u) >> 3) - (e.cy0 >> 3) + 1u : 0u;
-    const float r0x = ffrom(q2.w), r0y = ffrom(q3.x);
-    e.zdx = ffrom(q3.y);
-    e.zdy = ffrom(q3.z);
+    const float r0x = ffrom(q3.x), r0y = ffrom(q3.y);
+    e.zdx = ffrom(q2.y);
+    e.zdy = ffrom(q2.z);
     const float sxf = (float)X0 - r0x, syf = (float)Y0 - r0y;
-    e.zc0 = e.zdx * sxf + e.zdy * syf + ffrom(q3.w);
+    e.zc0 = e.zdx * sxf + e.zdy * syf + ffrom(q2.w);
     e.low = 0xFFFFFFFEull - order;
     return e;
 }

@@ -105,14 +105,14 @@ struct FrameDev {
     uint32_t ndraws, nviews, total_bins, ntris;
     uint32_t bin_k, bin_size, clip_cap, entry_cap;
     uint32_t bin_log2, bin_klog2;  // log2 of bin_size and of bin_k (both powers of two)
-    uint4* rec_raster;     // 4 x uint4 per record: edges, bbox, r0, z plane
-    float* rec_shade;      // shade_stride floats per record: 1/w plane, then attribute planes 0-1 (stride 9)
-                           // or 0-3 (stride 15), each plane (dx, dy, value at v0)
-    uint32_t shade_stride;
+    uint4* rec_raster;     // 4 x uint4 per record: edges, bbox, z plane, then what shading needs of it: r0, the draw
+                           // index and 1/w at v0. Written only for slots that hold a primitive, as all of a record.
+    float4* rec_shade;     // shade_quads x float4 per record: 1/w's dx and dy, then attribute planes 0-1 (2 quads) or
+                           // 0-3 (4 quads), each plane (dx, dy, value at v0)
+    uint32_t shade_quads;
     float4* rec_ext;       // 3 x float4 per record: attribute planes 4-7 (wide frames only)
     const SponzaDev* sponza;  // SponzaShader constants (wide frames only)
     const uint32_t* sched_gate;  // learned order: [1] != 0 on frames that predict and record (else null)
-    uint32_t* rec_meta;    // draw index (written only for slots that hold a primitive)
     uint2* clip_queue;     // per triangle routed to the clipper: (global triangle id, draw index), kClipLists lists
     uint32_t* clip_base;   // per global triangle: first fan record (relative to ntris)
     uint32_t* clip_order;  // per fan record: order key

@@ -106,9 +106,9 @@ __device__ __forceinline__ void bin_predict_one(const FrameDev& F, const MlpLds&
     if (lane < ns) {
         const uint32_t e = (uint32_t)(((uint64_t)lane * cnt) / ns);
         const uint32_t rec = F.entries[beg + e];
-        const uint4 q0 = F.rec_raster[(size_t)rec * 4], q2 = F.rec_raster[(size_t)rec * 4 + 2];
-        const uint4 q3 = F.rec_raster[(size_t)rec * 4 + 3];
-        const int32_t xmin = q2.y & 0x3FFF, xmax = (q2.y >> 16) & 0x3FFF, ymin = q2.z & 0x3FFF, ymax = (q2.z >> 16) & 0x3FFF;
+        const uint4 q0 = F.rec_raster[(size_t)rec * 4], q1 = F.rec_raster[(size_t)rec * 4 + 1];
+        const uint4 q2 = F.rec_raster[(size_t)rec * 4 + 2], q3 = F.rec_raster[(size_t)rec * 4 + 3];
+        const int32_t xmin = q1.w & 0x3FFF, xmax = (q1.w >> 16) & 0x3FFF, ymin = q2.x & 0x3FFF, ymax = (q2.x >> 16) & 0x3FFF;
         // bounding box inside the bin (pixels, ends exclusive)
         const int32_t bx0 = max(xmin - X0, (int32_t)sx0), bx1 = min(xmax - X0 + 1, (int32_t)(sx0 + S));
         const int32_t by0 = max(ymin - Y0, (int32_t)sy0), by1 = min(ymax - Y0 + 1, (int32_t)(sy0 + S));
@@ -117,9 +117,9 @@ __device__ __forceinline__ void bin_predict_one(const FrameDev& F, const MlpLds&
         const float tri = (float)max(0, (int32_t)(q0.x + q0.y + q0.z)) * (1.0f / 512.0f);
         area = fminf(tri, box);
         // depth over the box corners: z = zdx (x - r0x) + zdy (y - r0y) + z0
-        const float zdx = ffrom(q3.y), zdy = ffrom(q3.z);
-        const float ux = (float)(X0 + bx0) - ffrom(q2.w), uy = (float)(Y0 + by0) - ffrom(q3.x);
-        const float za = zdx * ux + zdy * uy + ffrom(q3.w);
+        const float zdx = ffrom(q2.y), zdy = ffrom(q2.z);
+        const float ux = (float)(X0 + bx0) - ffrom(q3.x), uy = (float)(Y0 + by0) - ffrom(q3.y);
+        const float za = zdx * ux + zdy * uy + ffrom(q2.w);
         const float wx = zdx * (float)max(0, bx1 - bx0), wy = zdy * (float)max(0, by1 - by0);
         const float z0 = fminf(za, za + wx) + fminf(0.0f, wy), z1 = fmaxf(za, za + wx) + fmaxf(0.0f, wy);
         if (z0 == z0 && z1 == z1 && z1 - z0 < 1.0e30f) {
@@ -128,13 +128,13 @@ __device__ __forceinline__ void bin_predict_one(const FrameDev& F, const MlpLds&
             zext = z1 - z0;
         }
         // mip level from the uv planes at the first vertex (slots 0 and 1)
-        const float* Sp = F.rec_shade + (size_t)rec * F.shade_stride;
-        const float4 s0 = make_float4(Sp[0], Sp[1], Sp[2], Sp[3]), s1 = make_float4(Sp[4], Sp[5], Sp[6], Sp[7]);
-        const DrawDev& D = F.draws[F.rec_meta[rec]];
+        const float4* Sp = F.rec_shade + (size_t)rec * F.shade_quads;
+        const float4 s0 = Sp[0], s1 = Sp[1];
+        const DrawDev& D = F.draws[q3.z];
         const uint32_t ti = D.tex_info;
         if (ti && D.deriv_slot == 0) {
-            const float g = fmaxf(fmaxf(fabsf(s0.w), fabsf(s1.x)), fmaxf(fabsf(s1.z), fabsf(s1.w))) /
-                            fmaxf(fabsf(s0.z), 1.0e-30f) * (float)(1u << (ti & 31u));
+            const float g = fmaxf(fmaxf(fabsf(s0.z), fabsf(s0.w)), fmaxf(fabsf(s1.y), fabsf(s1.z))) /
+                            fmaxf(fabsf(ffrom(q3.w)), 1.0e-30f) * (float)(1u << (ti & 31u));
             const float m = g > 1.0f ? __log2f(g) : 0.0f;
             mip = m == m ? fminf(m, (float)((ti >> 8) ? (ti >> 8) - 1u : 0u)) : 0.0f;
             textured = 1.0f;

@@ -255,10 +255,10 @@ struct srg_ctx {
     size_t h_tables_cap = 0;
     // arenas
     DevArray<uint4> rec_raster;
-    DevArray<float> rec_shade;
+    DevArray<float4> rec_shade;
     DevArray<float4> rec_ext;         // attribute planes 4-7, frames with a SponzaShader draw
     SponzaDev sponza{};               // SponzaShader constants (srg_set_sponza_constants)
-    DevArray<uint32_t> rec_meta, clip_base, clip_order;
+    DevArray<uint32_t> clip_base, clip_order;
     DevArray<uint2> clip_queue;
     DevArray<uint32_t> bin_count, bin_start, part_count, part_off, queue, queue2, entries, pairs, scan_blk;
     DevArray<uint16_t> order_bkt;   // per queue entry: its cost bucket
@@ -763,9 +763,9 @@ void tune_after_frame(srg_ctx* ctx, uint64_t sig, float ms)
 struct FrameArenas {
     uint8_t* tables = nullptr;
     uint4* rec_raster = nullptr;
-    float* rec_shade = nullptr;
+    float4* rec_shade = nullptr;
     float4* rec_ext = nullptr;
-    uint32_t *rec_meta = nullptr, *clip_base = nullptr, *clip_order = nullptr;
+    uint32_t *clip_base = nullptr, *clip_order = nullptr;
     uint2* clip_queue = nullptr;
     uint32_t *bin_count = nullptr, *bin_start = nullptr, *part_count = nullptr, *pairs = nullptr;
     uint32_t *part_off = nullptr, *queue = nullptr, *queue2 = nullptr, *entries = nullptr, *scan_blk = nullptr;
@@ -972,11 +972,11 @@ int run_frame(srg_ctx* ctx, bool noalloc)
             }
     }
     if (total_tris >= (1ull << 29)) return SRG_ERR_INVALID;  // order key is (triangle << 3) | fan
-    // setup records keep two attribute planes (9 floats of shade record) when
-    // no draw of the frame reads more, four (15 floats) otherwise; planes 4-7
+    // setup records keep two attribute planes (two quads of shade record) when
+    // no draw of the frame reads more, four (four quads) otherwise; planes 4-7
     // of a frame with a SponzaShader draw go to rec_ext
     const bool narrow = !wide && max_slots <= 2;
-    const uint32_t shade_stride = narrow ? 9u : 15u;
+    const uint32_t shade_quads = narrow ? 2u : 4u;
     const uint32_t NT = (uint32_t)total_tris;
 
     size_t off = 0;
@@ -1061,8 +1061,7 @@ int run_frame(srg_ctx* ctx, bool noalloc)
             // records first; the entry lists take what the scratch has left
             Carver R = C;
             A.rec_raster = R.take<uint4>(nrec * 4);
-            A.rec_shade = R.take<float>(nrec * shade_stride);
-            A.rec_meta = R.take<uint32_t>(nrec);
+            A.rec_shade = R.take<float4>(nrec * shade_quads);
             A.clip_order = R.take<uint32_t>(want_clip);
             A.rec_ext = wide ? R.take<float4>(nrec * 3) : nullptr;
             // each entry takes 4 bytes of list and 18 of (record, key, slot)
@@ -1075,8 +1074,8 @@ int run_frame(srg_ctx* ctx, bool noalloc)
             A.pairs = R.take<uint32_t>(3 * (want_entries + want_entries / 2));
             if (!R.ok) return SRG_ERR_OVERFLOW;
         } else {
-            if ((st = ctx->rec_raster.ensure(nrec * 4)) || (st = ctx->rec_shade.ensure(nrec * shade_stride)) ||
-                (st = ctx->rec_meta.ensure(nrec)) || (st = ctx->clip_order.ensure(want_clip)) ||
+            if ((st = ctx->rec_raster.ensure(nrec * 4)) || (st = ctx->rec_shade.ensure(nrec * shade_quads)) ||
+                (st = ctx->clip_order.ensure(want_clip)) ||
                 (st = ctx->entries.ensure(want_entries)) || (st = ctx->pairs.ensure(3 * (want_entries + want_entries / 2))) ||
                 (wide && (st = ctx->rec_ext.ensure(nrec * 3))))
                 return st;
@@ -1084,7 +1083,6 @@ int run_frame(srg_ctx* ctx, bool noalloc)
             ctx->entry_cap = (uint32_t)want_entries;
             A.rec_raster = ctx->rec_raster.ptr;
             A.rec_shade = ctx->rec_shade.ptr;
-            A.rec_meta = ctx->rec_meta.ptr;
             A.clip_order = ctx->clip_order.ptr;
             A.entries = ctx->entries.ptr;
             A.pairs = ctx->pairs.ptr;
@@ -1111,10 +1109,9 @@ int run_frame(srg_ctx* ctx, bool noalloc)
         F.entry_cap = (uint32_t)want_entries;
         F.rec_raster = A.rec_raster;
         F.rec_shade = A.rec_shade;
-        F.shade_stride = shade_stride;
+        F.shade_quads = shade_quads;
         F.rec_ext = A.rec_ext;
         F.sponza = wide ? (const SponzaDev*)(A.tables + o_sponza) : nullptr;
-        F.rec_meta = A.rec_meta;
         F.clip_queue = A.clip_queue;
         F.clip_base = A.clip_base;
         F.clip_order = A.clip_order;
@@ -1492,7 +1489,6 @@ void srg_destroy(srg_ctx* ctx)
     ctx->rec_raster.release();
     ctx->rec_shade.release();
     ctx->rec_ext.release();
-    ctx->rec_meta.release();
     ctx->clip_queue.release();
     ctx->clip_base.release();
     ctx->clip_order.release();
