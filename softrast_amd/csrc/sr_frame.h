@@ -94,6 +94,7 @@ struct SetupGroupDev {
     uint32_t nmembers;
 };
 constexpr uint32_t kMaxGroupMembers = 16;
+constexpr uint32_t kSetupSharedWaves = 16;  // resident waves of the shared set-up on a CU (128 VGPRs)
 
 struct FrameDev {
     const DrawDev* draws;

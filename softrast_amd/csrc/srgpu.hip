@@ -57,6 +57,36 @@ static uint64_t clip_pair_want(uint32_t clip_pairs)
     return (uint64_t)clip_pairs * 2 * kClipPairRegions * 5 / 4;
 }
 
+// Splits the lists of draws that share their geometry into setup groups,
+// larger ones first. A workgroup of k_setup sets its triangles up for every
+// draw of its group, one after another, so larger groups fetch less often and
+// run longer: with one group of twelve, 1080p / 1 M in twelve views was 3.8
+// rounds of resident workgroups, whose last, long round left a third of the
+// chip idle. So a group takes at most a quarter of the draws that a resident
+// wave will set up in all, and half of what its list has left: the launch ends
+// with short workgroups, which fill the gaps that the long ones leave. k_setup
+// with groups of up to sixteen in draw order -> now: twelve views of 1080p / 1 M
+// 377 -> 305 us, 64 of 512x512 / 100 k 177 -> 139, 8 / 16 / 64 of 1080p / 1 M
+// in eight draws 225 / 436 / 1,586 -> 203 / 388 / 1,572. At most an eighth or a
+// half instead of a quarter: 313 or 305, 145 or 140.
+static void split_groups(std::vector<std::vector<uint32_t>>& lists, const std::vector<DrawDev>& draws, uint32_t cus)
+{
+    uint64_t waves = 0;  // wave-draws of the shared lists
+    for (const auto& l : lists)
+        if (l.size() > 1) waves += (uint64_t)l.size() * ((draws[l[0]].ntris + 63u) / 64u);
+    if (!waves) return;
+    const size_t cap = (size_t)std::min<uint64_t>(std::max<uint64_t>(waves / (kSetupSharedWaves * cus * 4ull), 2), kMaxGroupMembers);
+    std::vector<std::vector<uint32_t>> out;
+    for (const auto& l : lists)
+        for (size_t at = 0; at < l.size();) {
+            const size_t left = l.size() - at, n = left <= 3 ? left : std::min(cap, (left + 1) / 2);
+            out.emplace_back(l.begin() + (ptrdiff_t)at, l.begin() + (ptrdiff_t)(at + n));
+            at += n;
+        }
+    std::stable_sort(out.begin(), out.end(), [](const auto& a, const auto& b) { return a.size() > b.size(); });
+    lists.swap(out);
+}
+
 // The frame's tables come along: `ntab` 16-byte words read from page-locked
 // host memory (a copy of their own is a launch more, about 3 us a frame).
 __global__ __launch_bounds__(256) void k_frame_init(uint32_t* counters, uint32_t* part_count, uint64_t* bin_cost,
@@ -912,7 +942,7 @@ int run_frame(srg_ctx* ctx, bool noalloc)
         total_tris += d.ntris;
     }
     // ---- setup groups: draws that share their geometry, at most
-    // kMaxGroupMembers each, in draw order ----
+    // kMaxGroupMembers each ----
     // groups of one first (k_setup<NS, false>), then the shared ones
     // (k_setup<NS, true>), each launch over its own range of workgroups
     std::vector<SetupGroupDev> gdev;
@@ -951,13 +981,13 @@ int run_frame(srg_ctx* ctx, bool noalloc)
             std::memcpy(key.f, fields, sizeof(fields));
             std::memcpy(key.slot_attr, d.slot_attr, sizeof(key.slot_attr));
             auto it = open_group.find(key);
-            if (it == open_group.end() || lists[it->second].size() >= kMaxGroupMembers) {
-                open_group[key] = (uint32_t)lists.size();
+            if (it == open_group.end()) {
+                it = open_group.emplace(key, (uint32_t)lists.size()).first;
                 lists.emplace_back();
-                it = open_group.find(key);
             }
             lists[it->second].push_back((uint32_t)i);
         }
+        split_groups(lists, ddev, (uint32_t)ctx->num_cus);
         for (int pass = 0; pass < 2; ++pass)
             for (const auto& l : lists) {
                 if ((l.size() > 1) != (pass == 1)) continue;
