@@ -1,6 +1,7 @@
 // sr_frame.h -- per-frame device tables shared by the front-end and back-end
 // kernels, and the wave-level helpers they use.
 #pragma once
+#include "sr_arena.h"
 #include "sr_device.h"
 
 namespace srg {
@@ -123,8 +124,8 @@ struct FrameDev {
     uint32_t* part_off;    // kBinParts x total_bins: first entry of a part of a bin's list
     uint32_t* entries;
     // (record, part-bin key, slot in the part's list) of every entry, as the
-    // count walks find them: three arrays of pair_total words, one after
-    // another; k_scatter writes entries from them after the scan. Region r <
+    // count walks find them: three arrays of one layout (sr_arena.h), from
+    // which k_scatter writes the entries after the scan. Region r <
     // pair_regions (a power of two; k_setup's workgroup index mod
     // pair_regions) fills
     // [r * pair_region_cap, (r + 1) * pair_region_cap) through its own
@@ -134,9 +135,9 @@ struct FrameDev {
     // therefore get the same pairs every frame; k_clip takes its triangles in
     // queue order, so after a frame whose clip regions could not each hold
     // all of its clip pairs the host sizes them so (C_CLIP_PAIRS).
-    uint32_t* pairs;
+    uint32_t *pair_rec, *pair_key, *pair_slot;
     uint32_t* pair_count;
-    uint32_t pair_regions, pair_region_cap, clip_pair_cap, pair_total;
+    uint32_t pair_regions, pair_region_cap, clip_pair_cap;
     uint32_t* queue;
     uint64_t* bin_cost;    // optional per bin (s_memtime ticks)
     uint32_t* counters;
@@ -148,7 +149,13 @@ struct FrameDev {
 // walks of different workgroups do not contend on one address. A frame uses
 // as many regions as k_setup has workgroups, at most kPairRegions, so that
 // every region holds a share of the frame's pairs.
-constexpr uint32_t kPairRegions = 256, kClipPairRegions = 8, kPairStride = 16;
+constexpr uint32_t kPairStride = 16;
+// First pair of a region; a whole array has fewer than 2^32 (sr_arena.h).
+__device__ __forceinline__ uint32_t pair_region_first(const FrameDev& F, uint32_t region)
+{
+    return region < F.pair_regions ? region * F.pair_region_cap
+                                   : F.pair_regions * F.pair_region_cap + (region - F.pair_regions) * F.clip_pair_cap;
+}
 
 // The clipper's queue is kClipLists lists, each with a counter on a line of
 // its own (the second word of a pair region's), because atomics on one address

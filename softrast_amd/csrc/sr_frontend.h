@@ -292,12 +292,12 @@ __device__ __forceinline__ void walk_big(const FrameDev& F, uint32_t part, uint3
         }
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
-            const uint32_t i = base + 64u * k + lane_id(), p = first_p + at + i, np = F.pair_total;
+            const uint32_t i = base + 64u * k + lane_id(), p = first_p + at + i;
             if (i < n && at + i < cap) {
-                F.pairs[p] = act[k] ? rec : kNoPair;
+                F.pair_rec[p] = act[k] ? rec : kNoPair;
                 if (act[k]) {
-                    F.pairs[np + p] = key[k];
-                    F.pairs[2u * np + p] = slot[k];
+                    F.pair_key[p] = key[k];
+                    F.pair_slot[p] = slot[k];
                 }
             }
         }
@@ -349,8 +349,7 @@ __device__ __forceinline__ void walk_bins(const FrameDev& F, uint32_t bins_x, ui
     const uint32_t region =
         clip ? F.pair_regions + blockIdx.x % kClipPairRegions : blockIdx.x & (F.pair_regions - 1u);
     const uint32_t cap = clip ? F.clip_pair_cap : F.pair_region_cap;
-    const uint32_t first_p = clip ? F.pair_regions * F.pair_region_cap + (region - F.pair_regions) * F.clip_pair_cap
-                                  : region * F.pair_region_cap;
+    const uint32_t first_p = pair_region_first(F, region);
     const uint32_t part = bin_part();
     uint32_t pres = 0;
     if (lane == 0 && total_all) pres = atomicAdd(&F.pair_count[region * kPairStride], total_all);
@@ -389,11 +388,11 @@ __device__ __forceinline__ void walk_bins(const FrameDev& F, uint32_t bins_x, ui
         // inside the pass instead of right after the atomic)
         const uint32_t ri = readlane_u32(pin(pres), 0) + it;
         if (valid && ri < cap) {
-            const uint32_t p = first_p + ri, np = F.pair_total;
-            F.pairs[p] = act ? orec : kNoPair;
+            const uint32_t p = first_p + ri;
+            F.pair_rec[p] = act ? orec : kNoPair;
             if (act) {
-                F.pairs[np + p] = pkey;
-                F.pairs[2u * np + p] = slot;
+                F.pair_key[p] = pkey;
+                F.pair_slot[p] = slot;
             }
         }
     }
@@ -1122,19 +1121,16 @@ __global__ __launch_bounds__(256) void k_scatter(FrameDev F, uint32_t chunk)
     if (F.counters[C_FLAGS] & (FLAG_ENTRY_OVERFLOW | FLAG_CLIP_OVERFLOW)) return;
     const uint32_t region = blockIdx.x;
     const uint32_t n = F.pair_count[region * kPairStride];  // within the region's capacity without overflow
-    const uint32_t first_p = region < F.pair_regions
-                                 ? region * F.pair_region_cap
-                                 : F.pair_regions * F.pair_region_cap + (region - F.pair_regions) * F.clip_pair_cap;
-    const uint32_t np = F.pair_total;
+    const uint32_t first_p = pair_region_first(F, region);
     const uint32_t nchunks = n / chunk + (n % chunk != 0u);
     for (uint32_t c = blockIdx.y; c < nchunks; c += gridDim.y) {
         for (uint32_t k = threadIdx.x; k < chunk; k += 256) {
             const uint32_t i = c * chunk + k;  // < n + chunk: no wrap for n < 2^32 - chunk
             if (i >= n) break;
             const uint32_t p = first_p + i;
-            const uint32_t rec = F.pairs[p];
+            const uint32_t rec = F.pair_rec[p];
             if (rec == kNoPair) continue;  // a candidate bin the corner test rejected
-            const uint32_t pkey = F.pairs[np + p], slot = F.pairs[2u * np + p];
+            const uint32_t pkey = F.pair_key[p], slot = F.pair_slot[p];
             F.entries[F.part_off[pkey] + slot] = rec;
         }
     }

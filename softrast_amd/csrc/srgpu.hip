@@ -1083,9 +1083,11 @@ int run_frame(srg_ctx* ctx, bool noalloc)
         want_clip = std::max<uint64_t>(want_clip, ctx->clip_cap);
         want_entries = std::max<uint64_t>(want_entries, ctx->entry_cap);
     }
+    if (want_entries > 0xFFFFFFF0ull) return SRG_ERR_OVERFLOW;
+    want_entries = std::min(want_entries, kMaxEntries);
 
     for (uint32_t attempt = 0;; ++attempt) {
-        if (want_clip > 0xFFFFFFF0ull - NT || want_entries > 0xFFFFFFF0ull) return SRG_ERR_OVERFLOW;
+        if (want_clip > 0xFFFFFFF0ull - NT) return SRG_ERR_OVERFLOW;
         const uint64_t nrec = (uint64_t)NT + want_clip;
         if (noalloc) {
             // records first; the entry lists take what the scratch has left
@@ -1099,14 +1101,14 @@ int run_frame(srg_ctx* ctx, bool noalloc)
             // all; 64 entries' worth is left for the alignment of the two
             const size_t left = R.left();
             if (!R.ok || left < (4096 + 64) * 22) return SRG_ERR_OVERFLOW;
-            want_entries = std::min<uint64_t>(left / 22 - 64, 0xFFFFFFF0ull);
+            want_entries = std::min<uint64_t>(left / 22 - 64, kMaxEntries);
             A.entries = R.take<uint32_t>(want_entries);
-            A.pairs = R.take<uint32_t>(3 * (want_entries + want_entries / 2));
+            A.pairs = R.take<uint32_t>(3 * pair_words(want_entries));
             if (!R.ok) return SRG_ERR_OVERFLOW;
         } else {
             if ((st = ctx->rec_raster.ensure(nrec * 4)) || (st = ctx->rec_shade.ensure(nrec * shade_quads)) ||
                 (st = ctx->clip_order.ensure(want_clip)) ||
-                (st = ctx->entries.ensure(want_entries)) || (st = ctx->pairs.ensure(3 * (want_entries + want_entries / 2))) ||
+                (st = ctx->entries.ensure(want_entries)) || (st = ctx->pairs.ensure(3 * pair_words(want_entries))) ||
                 (wide && (st = ctx->rec_ext.ensure(nrec * 3))))
                 return st;
             ctx->clip_cap = (uint32_t)want_clip;
@@ -1150,13 +1152,14 @@ int run_frame(srg_ctx* ctx, bool noalloc)
         F.part_count = A.part_count;
         F.part_off = A.part_off;
         F.entries = A.entries;
-        F.pairs = A.pairs;
+        const PairLayout P = pair_layout(want_entries, nblocks);
+        F.pair_rec = pair_array(A.pairs, P, 0);
+        F.pair_key = pair_array(A.pairs, P, 1);
+        F.pair_slot = pair_array(A.pairs, P, 2);
         F.pair_count = A.counters + kPairCounterBase;
-        // a power of two, so that k_setup finds its region with a mask
-        F.pair_regions = 1u << (31 - __builtin_clz(std::max<uint32_t>(1, std::min<uint32_t>(nblocks, kPairRegions))));
-        F.pair_region_cap = (uint32_t)(want_entries / F.pair_regions);
-        F.clip_pair_cap = (uint32_t)(want_entries / 2 / kClipPairRegions);
-        F.pair_total = F.pair_regions * F.pair_region_cap + kClipPairRegions * F.clip_pair_cap;
+        F.pair_regions = P.regions;
+        F.pair_region_cap = P.region_cap;
+        F.clip_pair_cap = P.clip_cap;
         F.queue = A.queue;
         F.bin_cost = A.bin_cost;
         F.counters = A.counters;
@@ -1342,11 +1345,14 @@ int run_frame(srg_ctx* ctx, bool noalloc)
             if (noalloc && (flags & FLAG_ENTRY_OVERFLOW)) return SRG_ERR_OVERFLOW;
             if (flags & FLAG_CLIP_OVERFLOW)
                 want_clip = std::max<uint64_t>(want_clip * 2, (uint64_t)ctx->h_counters[C_CLIPREC] + 64);
-            if (flags & FLAG_ENTRY_OVERFLOW)
-                want_entries = std::max({ want_entries * 2, (uint64_t)ctx->h_counters[C_ENTRIES] * 5 / 4,
-                                          (uint64_t)ctx->h_counters[C_PAIR_NEED] * F.pair_regions * 5 / 4,
-                                          (uint64_t)ctx->h_counters[C_CLIP_PAIR_NEED] * 2 * kClipPairRegions * 5 / 4,
-                                          clip_pair_want(ctx->h_counters[C_CLIP_PAIRS]) });
+            if (flags & FLAG_ENTRY_OVERFLOW) {
+                want_entries = grown_entries(
+                    want_entries, std::max({ (uint64_t)ctx->h_counters[C_ENTRIES] * 5 / 4,
+                                             (uint64_t)ctx->h_counters[C_PAIR_NEED] * F.pair_regions * 5 / 4,
+                                             (uint64_t)ctx->h_counters[C_CLIP_PAIR_NEED] * 2 * kClipPairRegions * 5 / 4,
+                                             clip_pair_want(ctx->h_counters[C_CLIP_PAIRS]) }));
+                if (!want_entries) return SRG_ERR_OVERFLOW;
+            }
             ctx->stats.retries++;
             continue;
         }
@@ -1355,7 +1361,7 @@ int run_frame(srg_ctx* ctx, bool noalloc)
         // could not hold all of them, the next frame sizes every region so
         // (the total is the same for the same triangles).
         if (!noalloc && clip_pair_want(ctx->h_counters[C_CLIP_PAIRS]) > want_entries)
-            ctx->entry_cap = (uint32_t)std::min<uint64_t>(clip_pair_want(ctx->h_counters[C_CLIP_PAIRS]), 0xFFFFFFF0ull);
+            ctx->entry_cap = (uint32_t)std::min(clip_pair_want(ctx->h_counters[C_CLIP_PAIRS]), kMaxEntries);
         ctx->stats.tris_in = total_tris;
         ctx->stats.prims = ctx->h_counters[C_PRIMS];
         ctx->stats.bin_entries = ctx->h_counters[C_TILE_ENTRIES];
