@@ -96,8 +96,9 @@ typedef struct srg_config {
     uint32_t sched_retrain_interval; /* SRG_ORDER_LEARNED: retrain every N frames (0 = never) */
     uint32_t wg_per_tile;   /* workgroups sharing one work bin, each owning a strip of
                                bin_size / wg_per_tile rows: 1, 2 or 4 (0 = 1, but 2 or 4 for 32-pixel
-                               bins of a frame so small that the GPU holds all its strips at once,
-                               without autotuner, learned order and recorded costs). Valid layouts
+                               bins of a frame whose strips are then at most six per CU -- fewer with a
+                               small wg_per_cu, one per CU with SRG_CFG_STATS -- without autotuner,
+                               learned order and recorded costs). Valid layouts
                                (bin_size, wg_per_tile): (8,1) (16,1) (32,1|2|4) (64,1|2|4) */
     uint32_t autotune_frames;        /* SRG_CFG_AUTOTUNE: frames timed per layout (0 = 3) */
     uint32_t reserved[4];

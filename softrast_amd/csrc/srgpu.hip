@@ -268,7 +268,7 @@ struct srg_ctx {
     // and eight kept planes: its grid, which strides over the clip queue, is
     // no larger, so that every workgroup runs in the first round
     uint32_t clip_resident[3] = { 2048, 2048, 2048 };
-    // k_backend workgroups resident per CU, per layout and variant (0: not asked yet)
+    // k_backend workgroups resident per CU, per layout (kLayouts' order) and variant (backend_variant)
     uint32_t backend_resident[8][4] = {};
     hipStream_t stream = nullptr;
     hipStream_t copy_stream = nullptr;  // asynchronous blits
@@ -677,21 +677,18 @@ bool layout_valid(uint32_t bin_size, uint32_t parts)
 // first item is its own index, so one that had to wait for a place would keep
 // an early, long item waiting: 2,048 workgroups where 1,536 fit took the 4K /
 // 2 M clustered frame from 580 to 645 us), no more than strips.
+uint32_t backend_variant(bool stats, bool wide) { return (wide ? 2u : 0u) + (stats ? 1u : 0u); }
+
+uint32_t backend_wg_per_cu(const srg_ctx* ctx, uint32_t resident)
+{
+    return ctx->cfg.wg_per_cu ? std::min(ctx->cfg.wg_per_cu, resident) : resident;
+}
+
 template <uint32_t S, uint32_t H, bool STATS, bool WIDE>
-void launch_backend_t(srg_ctx* ctx, uint32_t& resident, const FrameDev& F, hipEvent_t stop)
+void launch_backend_t(srg_ctx* ctx, uint32_t resident, const FrameDev& F, hipEvent_t stop)
 {
     constexpr uint32_t T = backend_threads(S, H);
-    if (!resident) {
-        int per_cu = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                &per_cu, reinterpret_cast<const void*>(&k_backend<S, H, STATS, WIDE>), (int)T, 0) != hipSuccess ||
-            per_cu <= 0) {
-            (void)hipGetLastError();
-            per_cu = 4;
-        }
-        resident = (uint32_t)per_cu;
-    }
-    const uint32_t wg = ctx->cfg.wg_per_cu ? std::min(ctx->cfg.wg_per_cu, resident) : resident;
+    const uint32_t wg = backend_wg_per_cu(ctx, resident);
     const uint32_t grid = std::min((uint32_t)ctx->num_cus * wg, std::max(1u, F.total_bins * (S / H)));
     if (stop)
         hipExtLaunchKernelGGL((k_backend<S, H, STATS, WIDE>), dim3(grid), dim3(T), 0, ctx->stream, nullptr, stop, 0, F);
@@ -700,15 +697,71 @@ void launch_backend_t(srg_ctx* ctx, uint32_t& resident, const FrameDev& F, hipEv
 }
 
 template <uint32_t S, uint32_t H>
-void launch_backend_t(srg_ctx* ctx, uint32_t resident[4], bool stats, const FrameDev& F, hipEvent_t stop)
+void launch_backend_t(srg_ctx* ctx, const uint32_t resident[4], bool stats, const FrameDev& F, hipEvent_t stop)
 {
+    const uint32_t r = resident[backend_variant(stats, F.rec_ext != nullptr)];
     if (F.rec_ext) {
-        if (stats) launch_backend_t<S, H, true, true>(ctx, resident[3], F, stop);
-        else launch_backend_t<S, H, false, true>(ctx, resident[2], F, stop);
+        if (stats) launch_backend_t<S, H, true, true>(ctx, r, F, stop);
+        else launch_backend_t<S, H, false, true>(ctx, r, F, stop);
     } else {
-        if (stats) launch_backend_t<S, H, true, false>(ctx, resident[1], F, stop);
-        else launch_backend_t<S, H, false, false>(ctx, resident[0], F, stop);
+        if (stats) launch_backend_t<S, H, true, false>(ctx, r, F, stop);
+        else launch_backend_t<S, H, false, false>(ctx, r, F, stop);
     }
+}
+
+template <uint32_t S, uint32_t H>
+void ask_backend_resident(uint32_t resident[4])
+{
+    const void* k[4] = {};
+    k[backend_variant(false, false)] = reinterpret_cast<const void*>(&k_backend<S, H, false, false>);
+    k[backend_variant(true, false)] = reinterpret_cast<const void*>(&k_backend<S, H, true, false>);
+    k[backend_variant(false, true)] = reinterpret_cast<const void*>(&k_backend<S, H, false, true>);
+    k[backend_variant(true, true)] = reinterpret_cast<const void*>(&k_backend<S, H, true, true>);
+    for (int i = 0; i < 4; ++i) {
+        int per_cu = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k[i], (int)backend_threads(S, H), 0) != hipSuccess ||
+            per_cu <= 0) {
+            (void)hipGetLastError();
+            per_cu = 4;
+        }
+        resident[i] = (uint32_t)per_cu;
+    }
+}
+
+// Asked once, by srg_create: a frame's layout depends on it, and a frame may
+// be launched into a stream capture.
+void ask_backend_resident(uint32_t (*r)[4])
+{
+    ask_backend_resident<8, 8>(r[0]);
+    ask_backend_resident<16, 16>(r[1]);
+    ask_backend_resident<32, 32>(r[2]);
+    ask_backend_resident<32, 16>(r[3]);
+    ask_backend_resident<32, 8>(r[4]);
+    ask_backend_resident<64, 64>(r[5]);
+    ask_backend_resident<64, 32>(r[6]);
+    ask_backend_resident<64, 16>(r[7]);
+}
+
+// Strips a frame of 32-pixel bins may be split into, where the configuration
+// leaves the split open: with more strips than bins each workgroup has less to
+// do in a row. k_backend with 1 / 2 / 4 strips a bin:
+//   two-plane frames: 320x180 (60 bins) 40 / 29 / 23 us, 960x540 (540) 29 / 24
+//     / 36, 1024x704 (704) 30 / 25 / 43, 1152x720 (864) 31 / 33 / 50: up to the
+//     six strips a CU that are resident;
+//   SponzaShader frames, of which four are resident: 960x540 42 / 36 / 40,
+//     1024x704 46 / 42 / 49, 1152x720 49 / 47 / 57: up to six as well, the
+//     last ones from the queue;
+//   a configured wg_per_cu of 1 and 2: 640x360 (240) 31 / 31 / 34 and 30 / 23
+//     / 25: up to one and a half rounds of the launched workgroups;
+//   statistics frames, every wave of which ends with an atomic on one address:
+//     256x256 (64) 25 / 19 / 22 with 10 k triangles, 62 / 46 / 36 with 250 k,
+//     320x180 42 / 32 / 27, 512x512 (256) 27 / 36 / 58 and 39 / 43 / 65,
+//     960x540 43 / 75 / 85: up to one strip a CU.
+uint64_t strip_limit(const srg_ctx* ctx, uint32_t parts, bool stats, bool wide)
+{
+    if (stats) return (uint64_t)ctx->num_cus;
+    const uint32_t wg = backend_wg_per_cu(ctx, ctx->backend_resident[parts == 2 ? 3 : 4][backend_variant(false, wide)]);
+    return (uint64_t)ctx->num_cus * std::min(6u, wg + wg / 2u);
 }
 
 // k_setup over the frame's setup groups: groups [0, nsingle) of one draw
@@ -727,7 +780,7 @@ void launch_setup(srg_ctx* ctx, const FrameDev& F, uint32_t nsingle, uint32_t si
 int launch_backend(srg_ctx* ctx, BackendLayout L, const FrameDev& F, hipEvent_t stop)
 {
     const bool stats = (F.flags & FF_STATS) != 0;
-    uint32_t(*r)[4] = ctx->backend_resident;
+    const uint32_t(*r)[4] = ctx->backend_resident;
     switch (L.bin_size * 8u + L.parts) {
     case 8 * 8 + 1: launch_backend_t<8, 8>(ctx, r[0], stats, F, stop); break;
     case 16 * 8 + 1: launch_backend_t<16, 16>(ctx, r[1], stats, F, stop); break;
@@ -874,16 +927,6 @@ int run_frame(srg_ctx* ctx, bool noalloc)
         total_bins += (uint64_t)v.bins_x * v.bins_y;
     }
     if (total_bins * kBinParts >= 0xFFFFFFF0ull) return SRG_ERR_INVALID;  // (part, bin) indices are 32-bit
-    // A frame with so few bins that the GPU holds all their strips at once is
-    // split further where the configuration leaves it open: each workgroup
-    // then has less to do in a row. k_backend with 1 / 2 / 4 strips a bin:
-    // 320x180 (60 bins) 17.4 / 12.2 / 9.7 us, 960x540 (540) 54 / 39 / 38; past
-    // what is resident it loses: 1280x720 (960) 22 / 29 / 49, 1080p (2,040,
-    // 250 k triangles) 53 / 59 / 103. Recorded bin costs belong to one layout.
-    if (!ctx->cfg.wg_per_tile && L.bin_size == 32 && !autotune && ctx->cfg.tile_order != SRG_ORDER_LEARNED &&
-        !(ctx->cfg.flags & SRG_CFG_TILE_COSTS))
-        while (L.parts < 4 && total_bins * L.parts * 2 <= (uint64_t)ctx->num_cus * backend_min_waves(32, 32, false, false))
-            L.parts *= 2;
 
     // ---- draws, textures, front-end blocks ----
     std::vector<DrawDev> ddev(ctx->draws.size());
@@ -941,6 +984,12 @@ int run_frame(srg_ctx* ctx, bool noalloc)
         std::memcpy(d.mvp, s.mvp, sizeof(d.mvp));
         total_tris += d.ntris;
     }
+    // Recorded bin costs belong to one layout.
+    if (!ctx->cfg.wg_per_tile && L.bin_size == 32 && !autotune && ctx->cfg.tile_order != SRG_ORDER_LEARNED &&
+        !(ctx->cfg.flags & SRG_CFG_TILE_COSTS))
+        while (L.parts < 4 &&
+               total_bins * L.parts * 2 <= strip_limit(ctx, L.parts * 2, (ctx->cfg.flags & SRG_CFG_STATS) != 0, wide))
+            L.parts *= 2;
     // ---- setup groups: draws that share their geometry, at most
     // kMaxGroupMembers each ----
     // groups of one first (k_setup<NS, false>), then the shared ones
@@ -1478,6 +1527,7 @@ int srg_create(const srg_config* cfg, srg_ctx** out)
                 ctx->clip_resident[i] = (uint32_t)per_cu * (uint32_t)ctx->num_cus;
         }
     }
+    ask_backend_resident(ctx->backend_resident);
     if (hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) { delete ctx; return SRG_ERR_HIP; }
     if (hipStreamCreateWithFlags(&ctx->copy_stream, hipStreamNonBlocking) != hipSuccess) {
         srg_destroy(ctx);
