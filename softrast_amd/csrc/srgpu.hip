@@ -57,8 +57,13 @@ static uint64_t clip_pair_want(uint32_t clip_pairs)
     return (uint64_t)clip_pairs * 2 * kClipPairRegions * 5 / 4;
 }
 
-// Splits the lists of draws that share their geometry into setup groups,
-// larger ones first. A workgroup of k_setup sets its triangles up for every
+// Draws [at, at + n) of a list of draws that share their geometry.
+struct GroupSpan {
+    uint32_t list, at, n;
+};
+
+// Splits the lists of draws that share their geometry into setup groups: those
+// of one draw first, then larger ones before smaller ones. A workgroup of k_setup sets its triangles up for every
 // draw of its group, one after another, so larger groups fetch less often and
 // run longer: with one group of twelve, 1080p / 1 M in twelve views was 3.8
 // rounds of resident workgroups, whose last, long round left a third of the
@@ -68,23 +73,36 @@ static uint64_t clip_pair_want(uint32_t clip_pairs)
 // with groups of up to sixteen in draw order -> now: twelve views of 1080p / 1 M
 // 377 -> 305 us, 64 of 512x512 / 100 k 177 -> 139, 8 / 16 / 64 of 1080p / 1 M
 // in eight draws 225 / 436 / 1,586 -> 203 / 388 / 1,572. At most an eighth or a
-// half instead of a quarter: 313 or 305, 145 or 140.
-static void split_groups(std::vector<std::vector<uint32_t>>& lists, const std::vector<DrawDev>& draws, uint32_t cus)
+// half instead of a quarter: 313 or 305, 145 or 140. Groups are spans of their
+// lists, placed by size: a vector each, sorted, cost a frame of 20,000 small
+// draws about 300 us of host time.
+static std::vector<GroupSpan> split_groups(const std::vector<std::vector<uint32_t>>& lists,
+                                           const std::vector<DrawDev>& draws, uint32_t cus)
 {
     uint64_t waves = 0;  // wave-draws of the shared lists
     for (const auto& l : lists)
         if (l.size() > 1) waves += (uint64_t)l.size() * ((draws[l[0]].ntris + 63u) / 64u);
-    if (!waves) return;
     const size_t cap = (size_t)std::min<uint64_t>(std::max<uint64_t>(waves / (kSetupSharedWaves * cus * 4ull), 2), kMaxGroupMembers);
-    std::vector<std::vector<uint32_t>> out;
-    for (const auto& l : lists)
-        for (size_t at = 0; at < l.size();) {
-            const size_t left = l.size() - at, n = left <= 3 ? left : std::min(cap, (left + 1) / 2);
-            out.emplace_back(l.begin() + (ptrdiff_t)at, l.begin() + (ptrdiff_t)(at + n));
+    std::vector<GroupSpan> spans;
+    spans.reserve(lists.size());
+    size_t first[kMaxGroupMembers + 1] = {};  // of the groups of a size: how many, then where the next one goes
+    for (uint32_t k = 0; k < lists.size(); ++k)
+        for (size_t at = 0; at < lists[k].size();) {
+            const size_t left = lists[k].size() - at, n = left <= 3 ? left : std::min(cap, (left + 1) / 2);
+            spans.push_back({ k, (uint32_t)at, (uint32_t)n });
+            ++first[n];
             at += n;
         }
-    std::stable_sort(out.begin(), out.end(), [](const auto& a, const auto& b) { return a.size() > b.size(); });
-    lists.swap(out);
+    size_t next = first[1];
+    first[1] = 0;
+    for (size_t n = kMaxGroupMembers; n > 1; --n) {
+        const size_t count = first[n];
+        first[n] = next;
+        next += count;
+    }
+    std::vector<GroupSpan> out(spans.size());
+    for (const GroupSpan& s : spans) out[first[s.n]++] = s;
+    return out;
 }
 
 // The frame's tables come along: `ntab` 16-byte words read from page-locked
@@ -1036,19 +1054,19 @@ int run_frame(srg_ctx* ctx, bool noalloc)
             }
             lists[it->second].push_back((uint32_t)i);
         }
-        split_groups(lists, ddev, (uint32_t)ctx->num_cus);
-        for (int pass = 0; pass < 2; ++pass)
-            for (const auto& l : lists) {
-                if ((l.size() > 1) != (pass == 1)) continue;
-                const uint32_t nt = ddev[l[0]].ntris;
-                gdev.push_back({ nblocks, nt, (uint32_t)gmem.size(), (uint32_t)l.size() });
-                gmem.insert(gmem.end(), l.begin(), l.end());
-                nblocks += (nt + kSetupThreads - 1) / kSetupThreads;
-                if (pass == 0) {
-                    nsingle = (uint32_t)gdev.size();
-                    single_blocks = nblocks;
-                }
+        const std::vector<GroupSpan> groups = split_groups(lists, ddev, (uint32_t)ctx->num_cus);
+        gdev.reserve(groups.size());
+        for (const GroupSpan& s : groups) {
+            const auto members = lists[s.list].begin() + (ptrdiff_t)s.at;
+            const uint32_t nt = ddev[*members].ntris;
+            gdev.push_back({ nblocks, nt, (uint32_t)gmem.size(), s.n });
+            gmem.insert(gmem.end(), members, members + (ptrdiff_t)s.n);
+            nblocks += (nt + kSetupThreads - 1) / kSetupThreads;
+            if (s.n == 1) {
+                nsingle = (uint32_t)gdev.size();
+                single_blocks = nblocks;
             }
+        }
     }
     if (total_tris >= (1ull << 29)) return SRG_ERR_INVALID;  // order key is (triangle << 3) | fan
     // setup records keep two attribute planes (two quads of shade record) when
