@@ -351,6 +351,12 @@ namespace {
 // A texture workspace of at most this is kept for the context's next texture
 // (20 bytes a texel of the base level: up to 2048^2); a larger one is freed.
 constexpr size_t kTexWorkKeep = 96u << 20;
+// An asynchronous blit of at most this is written to page-locked memory by the
+// de-tile kernel itself, which is then on the link for under a microsecond.
+// Through device rows and the copy engine / written directly, the blit and the
+// wait for it: 1x1 85 / 70 us, 64x64 86 / 70, 128x64 (32 KiB) 79 / 67; 160x90
+// 77 through the rows.
+constexpr size_t kFewRowsBytes = 32u << 10;
 constexpr size_t kStageBytes = 512u << 10;  // of each of srg_ctx::stage's two chunks
 
 uint64_t new_handle(srg_ctx* ctx) { return ctx->next_handle++; }
@@ -1960,11 +1966,12 @@ int srg_blit_async(srg_ctx* ctx, srg_fb* fb, void* linear, uint32_t flags, void 
     const size_t npx = (size_t)fb->width * fb->height;
     uint32_t* dev = nullptr;
     const bool direct = classify_dst(linear, npx * 4, &dev) == HostDst::pinned;
+    const bool few = npx * 4 <= kFewRowsBytes;
     if (!direct && !p.pinned && hipHostMalloc((void**)&p.pinned, npx * 4, 0) != hipSuccess) {
         p.pinned = nullptr;
         return SRG_ERR_NOMEM;
     }
-    if (!p.rows && hipMalloc((void**)&p.rows, npx * 4) != hipSuccess) {
+    if (!few && !p.rows && hipMalloc((void**)&p.rows, npx * 4) != hipSuccess) {
         p.rows = nullptr;
         return SRG_ERR_NOMEM;
     }
@@ -1973,12 +1980,15 @@ int srg_blit_async(srg_ctx* ctx, srg_fb* fb, void* linear, uint32_t flags, void 
     // frames are ordered after it, and copied out by the second stream's copy
     // engine. A kernel that writes the rows over the host link itself holds up
     // every kernel of the next frame: a small kernel launched beside it was
-    // done after 151 us, as the 8.3 MB were, instead of 10 beside the copy.
-    launch_detile(ctx->stream, 256, p.colour, p.rows, fb, 0, fb->height, (flags & SRG_BLIT_BGRA) != 0, nullptr);
+    // done after 151 us, as the 8.3 MB were, instead of 10 beside the copy. Few
+    // rows are done sooner than a copy would start.
+    if (few && !direct) HIP_TRY(hipHostGetDevicePointer((void**)&dev, p.pinned, 0));
+    launch_detile(ctx->stream, 256, p.colour, few ? dev : p.rows, fb, 0, fb->height, (flags & SRG_BLIT_BGRA) != 0, nullptr);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(ctx->ev[3], ctx->stream));
     HIP_TRY(hipStreamWaitEvent(ctx->copy_stream, ctx->ev[3], 0));
-    HIP_TRY(hipMemcpyAsync(direct ? linear : p.pinned, p.rows, npx * 4, hipMemcpyDeviceToHost, ctx->copy_stream));
+    if (!few)
+        HIP_TRY(hipMemcpyAsync(direct ? linear : p.pinned, p.rows, npx * 4, hipMemcpyDeviceToHost, ctx->copy_stream));
     p.job = BlitJob{ linear, direct ? nullptr : p.pinned, npx * 4, on_finish, user };
     HIP_TRY(hipLaunchHostFunc(ctx->copy_stream, blit_host_fn, &p.job));
     HIP_TRY(hipEventRecord(p.blit_done, ctx->copy_stream));
