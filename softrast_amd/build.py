@@ -50,6 +50,7 @@ def build_gpu(extra=()):
     out = PKG / "libsrgpu.so"
     tmp = out.with_suffix(".so.tmp")
     _run([HIPCC, *HIP_FLAGS, *extra, "-o", str(tmp), str(CSRC / "srgpu.hip")])
+    build_rcp_check()  # together with the library: it checks device functions that the library ships
     os.replace(tmp, out)
     return out
 
@@ -80,7 +81,6 @@ def build_all():
     build_scene()
     build_gpu()
     build_copy_calib()
-    build_rcp_check()
 
 
 if __name__ == "__main__":
