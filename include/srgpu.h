@@ -335,7 +335,9 @@ int srg_texture_build_rgba8(const uint8_t* linear_rgba8, uint32_t width, uint32_
  * builds the tiled level 0 and, if calc_mips, every mip on the GPU, and
  * registers the result as a texture. The bytes equal what
  * srg_texture_build_rgba8 makes (each mip is stbir_resize_uint8 of the base
- * level, Texture.cpp:196). */
+ * level, Texture.cpp:196). Work memory of about 20 bytes a texel (12 above
+ * 5 million texels) is taken; at most 96 MiB of it is kept for the context's
+ * next texture, until srg_destroy. */
 int srg_texture_create_rgba8(srg_ctx* ctx, const uint8_t* linear_rgba8, uint32_t width, uint32_t height,
                              int calc_mips, srg_handle* out);
 /* A registered texture's tiled bytes and layout (TextureData's m_texels,

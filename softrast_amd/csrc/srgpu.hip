@@ -2364,12 +2364,22 @@ int srg_texture_create_rgba8(srg_ctx* ctx, const uint8_t* linear, uint32_t width
     if (!ctx || !out || !linear) return SRG_ERR_INVALID;
     int st = texture_layout(width, height, calc_mips, L);
     if (st) return st;
-    // the passes of every level, longest chains (highest levels) first
-    MipPasses px{}, py{};
-    uint32_t bx = 0, by = 0, smax = 0;
-    size_t nrows = 0;  // float4
+    // The passes of every level, longest chains (highest levels) first. The
+    // rows of a whole chain are about as many float4 as the base has texels,
+    // half of them level 1's: where the workspace is freed again, level 1
+    // follows by itself in the other levels' place (8192^2: 0.8 GiB instead of
+    // 1.3, 15.8 ms instead of 14.7; 4096^2 4.2 both).
+    struct Batch {
+        MipPasses px{}, py{};
+        uint32_t bx = 0, by = 0;
+        size_t rows = 0;  // float4
+    };
+    Batch batch[2];
+    uint32_t smax = 0;
     uint64_t zero_at = L.total;  // the levels with padding texels, the last of the chain
+    const bool apart = (size_t)width * height * 20 > kTexWorkKeep;
     for (uint32_t m = L.n; m-- > 1;) {
+        Batch& B = batch[apart && m == 1 ? 1 : 0];
         const uint32_t mw = std::max(1u, width >> m), mh = std::max(1u, height >> m);
         if (mw < 32 || mh < 32) zero_at = L.offs[m];
         auto pass = [&](MipPasses& P, uint32_t& block, uint32_t in_log2, uint32_t outs, uint32_t lines) {
@@ -2380,18 +2390,19 @@ int srg_texture_create_rgba8(srg_ctx* ctx, const uint8_t* linear, uint32_t width
             q.lines = lines;
             q.seg = std::max(1u, kMipSegTexels >> q.log2_scale);
             q.segs = (outs + q.seg - 1) / q.seg;
-            q.rows_at = (uint32_t)nrows;
+            q.rows_at = (uint32_t)B.rows;
             q.dst_at = L.offs[m] / 4;
             block += q.segs * ((lines + 15) / 16);
             smax = std::max(smax, q.log2_scale);
         };
-        pass(px, bx, L.wl, mw, height);
-        pass(py, by, L.hl, mh, mw);
-        nrows += (size_t)height * mw;
+        pass(B.px, B.bx, L.wl, mw, height);
+        pass(B.py, B.by, L.hl, mh, mw);
+        B.rows += (size_t)height * mw;
     }
     // one workspace: base image, rows, weights
     const size_t base_bytes = (size_t)width * height * 4, w_count = smax ? mip_weights_at(smax + 1) : 0;
-    const size_t rows_at = base_bytes, weights_at = rows_at + nrows * 16, work = weights_at + w_count * 16;
+    const size_t rows_at = base_bytes, weights_at = rows_at + std::max(batch[0].rows, batch[1].rows) * 16,
+                 work = weights_at + w_count * 16;
     Texture t;
     t.bytes = L.total;
     t.wlog2 = L.wl;
@@ -2419,8 +2430,12 @@ int srg_texture_create_rgba8(srg_ctx* ctx, const uint8_t* linear, uint32_t width
         mip_filters(smax, hw.data());
         if (hipMemcpyAsync(weights, hw.data(), w_count * 16, hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
             return cleanup(SRG_ERR_HIP);
-        hipLaunchKernelGGL(k_mip_rows, dim3(bx), dim3(64), 0, ctx->stream, base, width, px, weights, rows);
-        hipLaunchKernelGGL(k_mip_cols, dim3(by), dim3(64), 0, ctx->stream, rows, height, py, weights, (uint32_t*)t.dev);
+        for (const Batch& B : batch)
+            if (B.rows) {
+                hipLaunchKernelGGL(k_mip_rows, dim3(B.bx), dim3(64), 0, ctx->stream, base, width, B.px, weights, rows);
+                hipLaunchKernelGGL(k_mip_cols, dim3(B.by), dim3(64), 0, ctx->stream, rows, height, B.py, weights,
+                                   (uint32_t*)t.dev);
+            }
     }
     if (hipGetLastError() != hipSuccess || hipStreamSynchronize(ctx->stream) != hipSuccess) return cleanup(SRG_ERR_HIP);
     cleanup(SRG_OK);
