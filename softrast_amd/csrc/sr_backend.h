@@ -399,8 +399,8 @@ __device__ __forceinline__ void raster_items(unsigned long long* keys, const uin
         const float zdx = ffrom(o[11 * 64]), zdy = ffrom(o[12 * 64]), zc0 = ffrom(o[13 * 64]);
         const unsigned long long lw = (unsigned long long)pin(o[14 * 64]);
         const uint32_t k = it - (m >> 7);
-        const uint32_t cx0 = pc & 127u, cy0 = (pc >> 14) & 127u;
-        const bool tight = ((pc >> 28) & 1u) != 0;
+        const uint32_t cx0 = pc & 127u, cy0 = (pc >> 7) & 127u;
+        const bool tight = (pc >> 14) != 0;
         const uint32_t snp = pd >> 17;
         const uint32_t brow = __umul24(k, pd & 0x1FFFFu) >> 16;  // k < 512, magic < 2^17
         const uint32_t x = 2u * ((cx0 >> 1) + (k - brow * snp)), yb = (cy0 & ~7u) + 8u * brow;
@@ -488,8 +488,7 @@ __device__ __forceinline__ void raster_wave(unsigned long long* keys, const Entr
                                             uint32_t sy0, unsigned long long& frags, uint32_t* stage)
 {
     const uint32_t lane = lane_id();
-    const uint32_t cw = e.cx1 > e.cx0 ? e.cx1 - e.cx0 : 0u;
-    const uint32_t np = cw ? ((e.cx1 - 1u) >> 1) - (e.cx0 >> 1) + 1u : 0u;  // column pairs per block row
+    const uint32_t np = e.cx1 > e.cx0 ? ((e.cx1 - 1u) >> 1) - (e.cx0 >> 1) + 1u : 0u;  // column pairs per block row
     const uint32_t n = has ? e.nby * np : 0u;
     // depths over a tile stay finite when the plane's terms are below 1e30
     const bool finite = __builtin_fabsf(e.zc0) < 1.0e30f && __builtin_fabsf(e.zdx) < 1.0e30f && __builtin_fabsf(e.zdy) < 1.0e30f;
@@ -502,7 +501,7 @@ __device__ __forceinline__ void raster_wave(unsigned long long* keys, const Entr
     // or one more (np <= 64); the 1-ulp reciprocal gives one of the two
     const uint32_t npp = max(np, 1u);
     const uint32_t magic = (uint32_t)(65536.0f * __builtin_amdgcn_rcpf((float)npp)) + 1u;
-    const uint32_t pk_cand = e.cx0 | (cw << 7) | (e.cy0 << 14) | (e.cy1 << 21) | ((e.tight ? 1u : 0u) << 28);
+    const uint32_t pk_cand = e.cx0 | (e.cy0 << 7) | ((e.tight ? 1u : 0u) << 14);
     const uint32_t pk_div = magic | (npp << 17);
     // each lane's entry into the wave's staging area: items read their
     // owner's fields from there (a broadcast where lanes share an owner)
