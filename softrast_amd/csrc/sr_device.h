@@ -45,10 +45,15 @@ __device__ __forceinline__ float maxps(float a, float b) { return a > b ? a : b;
 // mantissa bits, the exponent scaled exactly. So they are computed with the
 // hardware's reciprocal and reciprocal square root instead of being looked
 // up: m set into the low bits, the instruction, a rounding constant, a mask.
-// Two of RCPPS's 2,048 values lie within 0.13 fp32 ulp of a rounding tie, on
-// either side of it; with m one ulp lower and the constant one lower than half
-// a unit every value comes out right. rcp_check.hip compares every cell at
-// every exponent with the recorded tables, on the device. The look-ups were
+// With the exact middle and half a unit one of RCPPS's 2,048 values comes out
+// wrong and three lie within 0.13 fp32 ulp of it; with m one ulp lower and the
+// constant one lower every value is right, as long as the reciprocal is rounded
+// up at the four cells (243, 392, 1984, 2047) whose exact reciprocal lies 0.36
+// to 0.48 ulp below the word needed. RSQRTPS has 0.19 ulp of room at its
+// tightest cell. Both instructions may be off by an ulp, so the arithmetic does
+// not carry this: it rests on how this GPU rounds there, which rcp_check.hip
+// pins by comparing every cell at every exponent with the recorded tables, on
+// the device. The look-ups were
 // gathers from memory, 48 a pixel in the SponzaShader.
 
 // For inputs known to be positive normal numbers (rcpps: biased exponent <=

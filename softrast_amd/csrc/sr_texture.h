@@ -8,7 +8,7 @@
 // (k_mip_rows), a vertical pass weights those rows into the level's texels,
 // encodes them and writes them at their tiled addresses (k_mip_cols), with
 // the same float operations in the same order as the library. Every level is
-// made by the same two launches.
+// made by the same two launches (level 1 of a large texture by two more).
 //
 // Sizes are powers of two, so a level is 2^s times smaller than the base
 // along an axis and its filter is the same for every output: input texel j
@@ -19,8 +19,8 @@
 // A sum over up to 4 * 2^s texels has one order, so a line (a row; in the
 // second pass a column) is a serial chain. A lane therefore walks a line's
 // texels once, in order, for one channel, with the four open outputs' sums in
-// registers: 16 lines x 4 channels a wave, the weights wave-uniform (scalar
-// loads), each texel decoded once for its four weights. Lines are cut into
+// registers: 16 lines x 4 channels a wave, the weights the same for all of
+// them (staged through LDS), each texel decoded once for its four weights. Lines are cut into
 // segments of whole outputs (at least 256 texels, plus the 3 * 2^s that the
 // neighbours share), so the low levels, which have the work, run as many
 // short chains and the high ones, which have 4 * 2^s taps but few outputs,

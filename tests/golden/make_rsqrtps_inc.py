@@ -1,8 +1,8 @@
 """Turn the recorded RSQRTPS fixture (rsqrtps_table.txt) into C initialiser lists.
 
 Writes oracle/rsqrtps_table.inc (used by the CPU oracle) and
-softrast_amd/csrc/rsqrtps_table.inc (compiled into the HIP library). Both hold
-the same 4096 words: bits of rsqrt(1 + i/2048) for i = 0..2047, then of
+softrast_amd/csrc/rsqrtps_table.inc (what rcp_check.hip holds the library's
+formula against, word for word). Both hold the same 4096 words: bits of rsqrt(1 + i/2048) for i = 0..2047, then of
 rsqrt(2 + i/1024), as observed on an Intel host (see gen_rsqrtps_table.c).
 tests/test_oracle_kat.py checks both against the fixture.
 """
